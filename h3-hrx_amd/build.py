@@ -21,7 +21,8 @@ CSRC = HERE / "csrc"
 INCLUDE = HERE.parent / "include"
 OUT = HERE / "libh3attn.so"
 OBJ = HERE / "_build"
-SOURCES = ["prepare.hip", "plain.hip", "attention.hip", "attention_hm.hip", "noalloc.hip", "gemm.hip",
+SOURCES = ["prepare.hip", "plain.hip", "attention.hip", "attention_hm.hip", "attention_split.hip",
+           "noalloc.hip", "gemm.hip",
            "abi.cpp", "stack.cpp",
            "tables.cpp", "vsa.hip", "vsa_host.cpp", "fp6.hip"]
 ARCH = "gfx950"
@@ -50,7 +51,8 @@ FLAGS = [
 # sees NaN operands, so it may drop the NaN-quieting canonicalisations IEEE mode otherwise adds
 # to every max; infinities stay honoured (masked keys are -inf). The quantizer files keep full
 # IEEE semantics.
-EXTRA = {"attention.hip": ["-fno-honor-nans"], "attention_hm.hip": ["-fno-honor-nans"]}
+EXTRA = {name: ["-fno-honor-nans"]
+         for name in ("attention.hip", "attention_hm.hip", "attention_split.hip")}
 
 
 def _compile(src: pathlib.Path, obj: pathlib.Path) -> None:

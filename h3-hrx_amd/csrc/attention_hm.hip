@@ -1211,6 +1211,59 @@ uint32_t workgroups_per_xcd(const Geometry& g) {
   return std::min(g.per_xcd, std::max(1u, device_cus() / 8));  // one workgroup per CU
 }
 
+// A self-attention call with geometry `g` (operands, tokens, rows, capacity, strides and, kTm, the
+// token-major pitches), divided between this kernel and k_attention_split as split_plan says. The
+// FP6 and INT8 head-major rows have the same pitches.
+template <bool kFp6, bool kTm>
+hipError_t launch_self(Geometry g, uint32_t heads, hipStream_t stream) {
+  const SplitPlan plan = split_plan(g.tokens, g.rows, heads, device_cus());
+  g.q_blocks = (g.rows + kBlockQ - 1) / kBlockQ;
+  g.total = g.q_blocks * heads;
+  if (plan.split) {  // the first main_blocks full blocks here
+    g.q_blocks = g.rows / kBlockQ;
+    g.total = plan.main_blocks;
+  }
+  if (g.total > 0) {
+    g.per_xcd = (g.total + 7) / 8;
+    // token-major operands: one workgroup per block at every length (the chained form would spill)
+    g.wpx = kTm ? g.per_xcd : workgroups_per_xcd(g);
+    const dim3 grid(g.wpx * 8);
+    if constexpr (kTm)
+      hipLaunchKernelGGL((k_attention_hm<false, false, false, true>), grid, dim3(kThreads), 0,
+                         stream, g);
+    else if (chain_blocks(g))
+      hipLaunchKernelGGL((k_attention_hm<false, true, kFp6>), grid, dim3(kThreads), 0, stream, g);
+    else
+      hipLaunchKernelGGL((k_attention_hm<false, false, kFp6>), grid, dim3(kThreads), 0, stream, g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!plan.split) return hipSuccess;
+  SplitOperands x{};
+  x.qi = g.qi;
+  x.qs = g.qs;
+  x.ki = g.ki;
+  x.ks = g.ks;
+  x.vt = g.vt;
+  x.out = g.out;
+  x.tokens = g.tokens;
+  x.rows = g.rows;
+  x.capacity = g.capacity;
+  x.out_stride = g.out_stride;
+  x.heads = heads;
+  x.kv_head_limit = g.kv_head_limit;
+  x.head_limit = g.head_limit;
+  x.k_row = kTm ? g.k_row : kRowBytes;
+  x.q_row = kTm ? g.q_row : kRowBytes;
+  x.k_head = x.q_head = kTm ? 128u : (uint64_t)g.capacity * kRowBytes;
+  x.ks_key = kTm ? g.ks_key : 1u;
+  x.ks_head = kTm ? g.ks_head : g.capacity;
+  x.qs_row = kTm ? g.qs_row : 1u;
+  x.qs_head = kTm ? 1u : g.capacity;
+  x.fp6 = kFp6;
+  return launch_attention_split(x, plan, stream);
+}
+
 }  // namespace
 
 hipError_t launch_attention_hm(const h3_attention_cfg& cfg, uint32_t token_count, uint32_t heads,
@@ -1228,17 +1281,9 @@ hipError_t launch_attention_hm(const h3_attention_cfg& cfg, uint32_t token_count
   g.rows = std::min(token_count, cfg.tokens);
   g.capacity = cfg.token_capacity;
   g.out_stride = cfg.out_stride;
-  g.q_blocks = (token_count + kBlockQ - 1) / kBlockQ;
   g.kv_head_limit = cfg.kv_stride / 128;
   g.head_limit = cfg.out_stride / 128;
-  g.total = g.q_blocks * heads;
-  g.per_xcd = (g.total + 7) / 8;
-  g.wpx = workgroups_per_xcd(g);
-  if (chain_blocks(g))
-    hipLaunchKernelGGL((k_attention_hm<false, true>), dim3(g.wpx * 8), dim3(kThreads), 0, stream, g);
-  else
-    hipLaunchKernelGGL((k_attention_hm<false, false>), dim3(g.wpx * 8), dim3(kThreads), 0, stream, g);
-  return hipGetLastError();
+  return launch_self<false, false>(g, heads, stream);
 }
 
 // attention_i8qk_family's token-major operands on this kernel: Q and K codes [token][stride],
@@ -1259,7 +1304,6 @@ hipError_t launch_attention_hm_tm(const h3_attention_cfg& cfg, uint32_t token_co
   g.rows = std::min(token_count, cfg.tokens);
   g.capacity = cfg.token_capacity;
   g.out_stride = cfg.out_stride;
-  g.q_blocks = (token_count + kBlockQ - 1) / kBlockQ;
   g.kv_head_limit = cfg.kv_stride / 128;
   g.head_limit = cfg.out_stride / 128;
   g.k_row = cfg.kv_stride;
@@ -1267,12 +1311,7 @@ hipError_t launch_attention_hm_tm(const h3_attention_cfg& cfg, uint32_t token_co
   g.qs_row = cfg.q_stride / 128;
   g.ks_key = ks_head_major ? 1u : g.kv_head_limit;
   g.ks_head = ks_head_major ? cfg.tokens : 1u;
-  g.total = g.q_blocks * heads;
-  g.per_xcd = (g.total + 7) / 8;
-  g.wpx = g.per_xcd;  // one workgroup per block at every length (the chained form would spill)
-  hipLaunchKernelGGL((k_attention_hm<false, false, false, true>), dim3(g.wpx * 8), dim3(kThreads),
-                     0, stream, g);
-  return hipGetLastError();
+  return launch_self<false, true>(g, heads, stream);
 }
 
 hipError_t launch_attention_hm_fp6(const h3_attention_cfg& cfg, uint32_t token_count,
@@ -1290,19 +1329,9 @@ hipError_t launch_attention_hm_fp6(const h3_attention_cfg& cfg, uint32_t token_c
   g.rows = std::min(token_count, cfg.tokens);
   g.capacity = cfg.token_capacity;
   g.out_stride = cfg.out_stride;
-  g.q_blocks = (token_count + kBlockQ - 1) / kBlockQ;
   g.kv_head_limit = cfg.kv_stride / 128;
   g.head_limit = cfg.out_stride / 128;
-  g.total = g.q_blocks * heads;
-  g.per_xcd = (g.total + 7) / 8;
-  g.wpx = workgroups_per_xcd(g);
-  if (chain_blocks(g))
-    hipLaunchKernelGGL((k_attention_hm<false, true, true>), dim3(g.wpx * 8), dim3(kThreads), 0,
-                       stream, g);
-  else
-    hipLaunchKernelGGL((k_attention_hm<false, false, true>), dim3(g.wpx * 8), dim3(kThreads), 0,
-                       stream, g);
-  return hipGetLastError();
+  return launch_self<true, false>(g, heads, stream);
 }
 
 hipError_t launch_attention_hm_cross(const h3_cross_cfg& cfg, const int32_t* qi, const float* qs,

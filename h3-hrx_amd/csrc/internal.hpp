@@ -96,6 +96,33 @@ hipError_t launch_attention_hm_fp6(const h3_attention_cfg& cfg, uint32_t token_c
                                    uint32_t heads, const void* qf, const float* qs, const void* kf,
                                    const float* ks, const uint16_t* vt, uint16_t* out,
                                    hipStream_t stream);
+// The same attention with a tile's keys split over the waves of a workgroup (attention_split.hip),
+// for the blocks that would leave most of the chip idle. How a call of `heads` rows is divided:
+// `main_blocks` full 256-query blocks (head-major order) on k_attention_hm; the full blocks after
+// them in units of qw_full 32-query tiles and the heads' last, partial blocks in units of qw_rest
+// tiles on k_attention_split. `split` false: everything on k_attention_hm.
+struct SplitPlan {
+  bool split;
+  uint32_t main_blocks, qw_full, qw_rest;
+};
+SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t cus);
+// Operands of k_attention_split in either layout: byte pitches of a token's code row and of a head
+// for K and Q, element pitches of a key's (query's) scale and of a head for the scales.
+struct SplitOperands {
+  const void* qi;
+  const float* qs;
+  const void* ki;
+  const float* ks;
+  const uint16_t* vt;
+  uint16_t* out;
+  uint32_t tokens, rows, capacity, out_stride, heads, kv_head_limit, head_limit;
+  uint32_t k_row, q_row;
+  uint64_t k_head, q_head;
+  uint32_t ks_key, ks_head, qs_row, qs_head;
+  bool fp6;
+};
+hipError_t launch_attention_split(const SplitOperands& x, const SplitPlan& plan,
+                                  hipStream_t stream);
 // Compute units of the current device (cached per device; 256 if the query fails).
 uint32_t device_cus();
 // attention_i8qkhm: the head-major INT8 kernel of attention_hm.hip (eight waves of 32 queries,
