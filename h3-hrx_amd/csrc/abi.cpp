@@ -224,7 +224,7 @@ int attention_common(const char* stage, const h3_attention_cfg* cfg, uint32_t to
                      uint32_t heads, h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt,
                      h3_view out, hipStream_t stream, int mode, float skip_tau = 0.0f,
                      h3_view routes = {}, h3_view lengths = {}, h3_view workspace = {},
-                     bool static_workspace = false) {
+                     bool static_workspace = false, const VsaPrefix& prefix = {}) {
   const bool head_major = mode == kModeHeadI8;
   const bool vsa = mode == kModeTokenI8Vsa;
   const bool fp6 = mode == kModeTokenI4Fp6;
@@ -301,7 +301,7 @@ int attention_common(const char* stage, const h3_attention_cfg* cfg, uint32_t to
                                                 static_cast<uint16_t*>(out.ptr),
                                                 static_cast<const int32_t*>(routes.ptr),
                                                 static_cast<const int32_t*>(lengths.ptr),
-                                                workspace.ptr, stream));
+                                                workspace.ptr, prefix, stream));
   }
   if ((st = device_ready(stage))) return st;
   if (fp6)
@@ -389,9 +389,46 @@ int attention_i8qk_static_ws(const h3_attention_cfg* cfg, uint32_t token_count, 
 
 int vsa_attention_i8_ws(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads,
                         h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt, h3_view out,
-                        h3_view routes, h3_view lengths, h3_view workspace, hipStream_t stream) {
+                        h3_view routes, h3_view lengths, h3_view workspace,
+                        const VsaPrefix& prefix, hipStream_t stream) {
   return attention_common("VSA attention", cfg, token_count, heads, qi, qs, ki, ks, vt, out,
-                          stream, kModeTokenI8Vsa, 0.0f, routes, lengths, workspace);
+                          stream, kModeTokenI8Vsa, 0.0f, routes, lengths, workspace, false,
+                          prefix);
+}
+
+int vsa_attention_f16(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads, h3_view q,
+                      h3_view k, h3_view v, h3_view out, h3_view routes, h3_view lengths,
+                      const VsaPrefix& prefix, hipStream_t stream) {
+  const char* stage = "VSA attention f16";
+  int st = check_attention_cfg(stage, cfg, token_count, heads);
+  if (st) return st;
+  // kernels/vsa_attention_16.loom:113-123, 584-587: blocks = tokens / 64 query cubes, routes
+  // [out_stride/128][blocks][blocks] i32, lengths [blocks] i32; q [token_capacity][q_stride],
+  // k and v [token_capacity][kv_stride], out [token_count][out_stride], all f16.
+  if (cfg->tokens % 64 != 0 || cfg->tokens / 64 > 16384)
+    return set_error(H3_ERR_CONFIG, "%s: tokens %u is not 64 * blocks with blocks <= 16384",
+                     stage, cfg->tokens);
+  const size_t cap = cfg->token_capacity, blocks = cfg->tokens / 64;
+  const TouchedHeads th = touched_heads(*cfg, heads);
+  if (th.q > cfg->q_stride / 128)
+    return set_error(H3_ERR_CONFIG, "%s: q_stride %u holds %u query heads, the launch reads %zu",
+                     stage, cfg->q_stride, cfg->q_stride / 128, th.q);
+  h3_view views[6] = {q, k, v, out, routes, lengths};
+  size_t need[6] = {cap * cfg->q_stride * 2,
+                    cap * cfg->kv_stride * 2,
+                    cap * cfg->kv_stride * 2,
+                    ((size_t)(token_count - 1) * cfg->out_stride + th.q * 128) * 2,
+                    th.q * blocks * blocks * 4,
+                    blocks * 4};
+  if ((st = check_bindings(stage, views, need, 6))) return st;
+  if ((st = check_aligned16(stage, {q, k, v}))) return st;  // 16-byte row loads
+  if ((st = device_ready(stage))) return st;
+  return launched(stage, launch_attention_vsa_f16(
+                             *cfg, token_count, heads, static_cast<const uint16_t*>(q.ptr),
+                             static_cast<const uint16_t*>(k.ptr),
+                             static_cast<const uint16_t*>(v.ptr), static_cast<uint16_t*>(out.ptr),
+                             static_cast<const int32_t*>(routes.ptr),
+                             static_cast<const int32_t*>(lengths.ptr), prefix, stream));
 }
 
 int vsa_gather_pool(const h3_vsa_cfg* cfg, h3_view src, h3_view lengths, h3_view x, h3_view y,
@@ -940,37 +977,8 @@ int h3_vsa_attention_i8(const h3_attention_cfg* cfg, uint32_t token_count, uint3
 int h3_vsa_attention_f16(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads,
                          h3_view q, h3_view k, h3_view v, h3_view out, h3_view routes,
                          h3_view lengths, h3_stream stream) {
-  const char* stage = "VSA attention f16";
-  int st = check_attention_cfg(stage, cfg, token_count, heads);
-  if (st) return st;
-  // kernels/vsa_attention_16.loom:113-123, 584-587: blocks = tokens / 64 query cubes, routes
-  // [out_stride/128][blocks][blocks] i32, lengths [blocks] i32; q [token_capacity][q_stride],
-  // k and v [token_capacity][kv_stride], out [token_count][out_stride], all f16.
-  if (cfg->tokens % 64 != 0 || cfg->tokens / 64 > 16384)
-    return set_error(H3_ERR_CONFIG, "%s: tokens %u is not 64 * blocks with blocks <= 16384",
-                     stage, cfg->tokens);
-  const size_t cap = cfg->token_capacity, blocks = cfg->tokens / 64;
-  const TouchedHeads th = touched_heads(*cfg, heads);
-  if (th.q > cfg->q_stride / 128)
-    return set_error(H3_ERR_CONFIG, "%s: q_stride %u holds %u query heads, the launch reads %zu",
-                     stage, cfg->q_stride, cfg->q_stride / 128, th.q);
-  h3_view views[6] = {q, k, v, out, routes, lengths};
-  size_t need[6] = {cap * cfg->q_stride * 2,
-                    cap * cfg->kv_stride * 2,
-                    cap * cfg->kv_stride * 2,
-                    ((size_t)(token_count - 1) * cfg->out_stride + th.q * 128) * 2,
-                    th.q * blocks * blocks * 4,
-                    blocks * 4};
-  if ((st = check_bindings(stage, views, need, 6))) return st;
-  if ((st = check_aligned16(stage, {q, k, v}))) return st;  // 16-byte row loads
-  if ((st = device_ready(stage))) return st;
-  return launched(stage, launch_attention_vsa_f16(
-                             *cfg, token_count, heads, static_cast<const uint16_t*>(q.ptr),
-                             static_cast<const uint16_t*>(k.ptr),
-                             static_cast<const uint16_t*>(v.ptr), static_cast<uint16_t*>(out.ptr),
-                             static_cast<const int32_t*>(routes.ptr),
-                             static_cast<const int32_t*>(lengths.ptr),
-                             reinterpret_cast<hipStream_t>(stream)));
+  return vsa_attention_f16(cfg, token_count, heads, q, k, v, out, routes, lengths, {},
+                           reinterpret_cast<hipStream_t>(stream));
 }
 
 int h3_vsa_attention_i8_ws(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads,
@@ -979,7 +987,7 @@ int h3_vsa_attention_i8_ws(const h3_attention_cfg* cfg, uint32_t token_count, ui
                            h3_stream stream) {
   if (!workspace.ptr) return null_workspace("VSA attention");
   return vsa_attention_i8_ws(cfg, token_count, heads, qi, qs, ki, ks, vt, out, routes, lengths,
-                             workspace, reinterpret_cast<hipStream_t>(stream));
+                             workspace, {}, reinterpret_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -138,6 +138,9 @@ struct Args {
   uint32_t blocks;         // k_attention_vsa: tokens / 64
   uint32_t base;           // k_attention_vsa: first (head, cube) item of this launch
   float scale;             // k_attention_vsa<·, true>: the score scale of the f16 operands
+  uint32_t cube0;          // k_attention_vsa: query cube of a head's first item
+  uint32_t splits;         // k_attention_vsa<·, ·, true>: items (key ranges) per query cube
+  float* part;             // ..., and their partial results (VsaPart)
 };
 
 __device__ __forceinline__ uint32_t swap23(uint32_t m) {
@@ -1157,11 +1160,65 @@ __device__ __forceinline__ void vsa_step(const char* kst, const char* vst, const
 
 __device__ __forceinline__ uint32_t rfl(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Query cubes that keep (nearly) every key cube: the prefix's. Their lists are several times a
+// video cube's (387 key cubes against 44 at 17,704 tokens behind a 154-token prefix, keep 10 %), and
+// a launch of one generation lasts as long as its longest list, so among the other cubes each of
+// them held up a whole generation (13 launches of 639 us there, 62 us without them). They go first,
+// in launches of their own, and where they are too few to fill the chip each is split: item
+// (cube, split) walks one range of the key cubes and writes its unnormalised O (f32 [64][128]) and
+// its rows' running max and sum, and k_vsa_combine weighs the ranges of a cube together.
+constexpr uint32_t kVsaPartO = 64 * 128;              // floats of an item's O
+constexpr uint32_t kVsaPart = kVsaPartO + 2 * 64;     // + m[64], l[64]
+__global__ __launch_bounds__(256) void k_vsa_combine(const float* __restrict__ part,
+                                                     uint16_t* __restrict__ out, uint32_t cubes,
+                                                     uint32_t splits, uint32_t rows,
+                                                     uint32_t out_stride, uint32_t kv_head_limit,
+                                                     uint32_t head_limit) {
+  const uint32_t item = blockIdx.x, head_y = item / cubes, cube = item % cubes;
+  const uint32_t head = head_y % kv_head_limit % head_limit;
+  const float* base = part + (size_t)item * splits * kVsaPart;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t piece = threadIdx.x + 256 * i;  // eight channels of a row
+    const uint32_t r = piece >> 4, chunk = piece & 15;
+    float top = -1.0e30f;
+    for (uint32_t s = 0; s < splits; ++s) top = fmaxf(top, base[s * kVsaPart + kVsaPartO + r]);
+    float sum[8] = {}, l = 0.0f;
+    for (uint32_t s = 0; s < splits; ++s) {
+      const float* p = base + s * kVsaPart;
+      const float w = __builtin_amdgcn_exp2f(p[kVsaPartO + r] - top);
+      const float4 a = *reinterpret_cast<const float4*>(p + 128 * r + 8 * chunk);
+      const float4 b = *reinterpret_cast<const float4*>(p + 128 * r + 8 * chunk + 4);
+      l = __builtin_fmaf(p[kVsaPartO + 64 + r], w, l);
+      sum[0] = __builtin_fmaf(a.x, w, sum[0]);
+      sum[1] = __builtin_fmaf(a.y, w, sum[1]);
+      sum[2] = __builtin_fmaf(a.z, w, sum[2]);
+      sum[3] = __builtin_fmaf(a.w, w, sum[3]);
+      sum[4] = __builtin_fmaf(b.x, w, sum[4]);
+      sum[5] = __builtin_fmaf(b.y, w, sum[5]);
+      sum[6] = __builtin_fmaf(b.z, w, sum[6]);
+      sum[7] = __builtin_fmaf(b.w, w, sum[7]);
+    }
+    const float inv = 1.0f / l;
+    const uint32_t q = 64 * cube + r;
+    if (q >= rows) continue;
+    uint16_t* dst = out + (size_t)q * out_stride + 128 * head + 8 * chunk;
+    // two 8-byte stores: the output binding is 8-byte aligned, as the unsplit cubes' stores need
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const v4h h = {(_Float16)(sum[4 * k] * inv), (_Float16)(sum[4 * k + 1] * inv),
+                     (_Float16)(sum[4 * k + 2] * inv), (_Float16)(sum[4 * k + 3] * inv)};
+      *reinterpret_cast<v4h*>(dst + 4 * k) = h;
+    }
+  }
+}
+
 // kHmScales: a.ks is head-major, [kv_head_limit][tokens]; otherwise token-major as the
 // operands' producer writes it, [tokens][kv_head_limit]. kF16: the f16 form (a.qi, a.ki, a.vt
 // are the token-major f16 q, k, v; a.q_row and a.kv_bytes their row pitches in bytes; scores
 // times a.scale), on two-stage rings so that four workgroups share a CU (35.1 KB of LDS each).
-template <bool kHmScales, bool kF16 = false>
+// kPart: the items are ranges of the key cubes, written as partial results (k_vsa_combine).
+template <bool kHmScales, bool kF16 = false, bool kPart = false>
 __global__ __launch_bounds__(kVsaThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_attention_vsa(Args a) {
   __shared__ __attribute__((aligned(16))) char k0s[vsa_kstage<kF16>()];
@@ -1178,9 +1235,12 @@ void k_attention_vsa(Args a) {
   const uint32_t b = blockIdx.x;
   const uint32_t local = (b & 7u) * a.per_xcd + (b >> 3);
   if (local >= a.total) return;
-  const uint32_t logical = a.base + local;
+  const uint32_t item = a.base + local;
+  const uint32_t logical = kPart ? item / a.splits : item;
   const uint32_t head_y = logical / a.q_blocks;
-  const uint32_t cube = logical % a.q_blocks;  // this workgroup's query cube
+  const uint32_t cube = a.cube0 + logical % a.q_blocks;  // this workgroup's query cube
+  const uint32_t split = kPart ? item % a.splits : 0u;
+  const uint32_t scan_end = kPart ? a.blocks * (split + 1) / a.splits : a.blocks;
   const uint32_t kv_head = head_y % a.kv_head_limit;
   const uint32_t head = kv_head % a.head_limit;
 
@@ -1233,21 +1293,21 @@ void k_attention_vsa(Args a) {
     const uint32_t kb = at + threadIdx.x;
     keep = 0;
     len = 0;
-    if (kb < a.blocks) {
+    if (kb < scan_end) {
       keep = route[kb];
       len = a.lengths[kb];
     }
   };
-  uint32_t scan = 0;  // first key cube not yet listed
-  while (scan < a.blocks) {
+  uint32_t scan = kPart ? a.blocks * split / a.splits : 0u;  // first key cube not yet listed
+  while (scan < scan_end) {
     // ---- list the live halves of the kept cubes from `scan` on, kVsaThreads cubes per pass
     uint32_t count = 0;
     int32_t keep_next, len_next;
     fetch(scan, keep_next, len_next);
-    while (scan < a.blocks) {
+    while (scan < scan_end) {
       const uint32_t kb = scan + threadIdx.x;
       const int32_t keep = keep_next, len = len_next;
-      if (scan + kVsaThreads < a.blocks) fetch(scan + kVsaThreads, keep_next, len_next);
+      if (scan + kVsaThreads < scan_end) fetch(scan + kVsaThreads, keep_next, len_next);
       const uint32_t live = keep == 0 ? 0u : len < 0 ? 0u : len > 64 ? 64u : (uint32_t)len;
       const uint64_t ball0 = __ballot(live > 0);
       const uint64_t ball1 = __ballot(live > (uint32_t)kVsaKeys);
@@ -1366,8 +1426,24 @@ void k_attention_vsa(Args a) {
     step_barrier<kWaitAll>();  // no staging load outlives the run; the stages are reused
   }
 
-  // ---- normalise and store rows < token_count
   const float l_tot = st.l + __shfl_xor(st.l, 32);
+  if constexpr (kPart) {  // the range's unnormalised O, max and sum
+    float* p = a.part + (size_t)item * kVsaPart;
+    const uint32_t r = wave * kQueriesPerWave + n;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(p + 128 * r + 32 * db + 8 * i + 4 * half) =
+            make_float4(st.acc[db][4 * i], st.acc[db][4 * i + 1], st.acc[db][4 * i + 2],
+                        st.acc[db][4 * i + 3]);
+    if (half == 0) {
+      p[kVsaPartO + r] = st.m;
+      p[kVsaPartO + 64 + r] = l_tot;
+    }
+    return;
+  }
+  // ---- normalise and store rows < token_count
   const float inv = 1.0f / l_tot;
   if (q < a.token_count && q < a.tokens) {
     uint16_t* dst = a.out + (size_t)q * a.out_stride + head * 128;
@@ -1653,11 +1729,61 @@ size_t scales_workspace_bytes(const h3_attention_cfg& cfg) {
   return (size_t)(cfg.kv_stride / 128) * cfg.tokens * 4;
 }
 
+// Workgroups of one generation of k_attention_vsa: four per CU.
+static uint32_t vsa_generation() { return std::max(1u, 4u * device_cus()); }
+
+size_t vsa_part_bytes(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t* splits) {
+  // As many ranges as fit one generation, each of at least eight key cubes and at most 16 of them
+  // (a range costs a 33 KB partial result): at 32 heads behind a 3-cube prefix, ten ranges of 39
+  // key cubes, whose walk is that of an ordinary cube there.
+  const uint32_t items = std::max(1u, heads * cubes);
+  *splits = cubes ? std::max(1u, std::min({vsa_generation() / items, 16u, blocks / 8})) : 1u;
+  return *splits > 1 ? (size_t)items * *splits * kVsaPart * 4 : 0;
+}
+
+// The launches of a call: the prefix's query cubes first, then the others, each one launch per
+// generation of resident workgroups: its workgroups start together and walk their ascending key
+// lists at about the same pace, so more of the tiles they share are still in L2 (measured at 129k
+// tokens with token-major scales: 45.9 ms against 56.5 ms for one launch of all the work).
+template <bool kHmScales, bool kF16>
+static hipError_t launch_vsa_cubes(Args a, uint32_t heads, const VsaPrefix& prefix,
+                                   hipStream_t stream) {
+  const uint32_t all = a.q_blocks, gen = vsa_generation();
+  auto generations = [&](uint32_t items, auto kernel) {
+    for (uint32_t base = 0; base < items; base += gen) {
+      a.base = base;
+      a.total = std::min(gen, items - base);
+      a.per_xcd = (a.total + 7) / 8;
+      hipLaunchKernelGGL(kernel, dim3(a.per_xcd * 8), dim3(kVsaThreads), 0, stream, a);
+    }
+  };
+  const uint32_t first = std::min(prefix.cubes, all);
+  if (first > 0) {
+    a.q_blocks = first;
+    a.splits = prefix.splits;
+    a.part = prefix.part;
+    if (prefix.splits > 1) {
+      if constexpr (kHmScales || kF16) {  // the runtime's two forms
+        generations(first * heads * prefix.splits, k_attention_vsa<kHmScales, kF16, true>);
+        hipLaunchKernelGGL(k_vsa_combine, dim3(first * heads), dim3(256), 0, stream, prefix.part,
+                           a.out, first, prefix.splits, std::min(a.token_count, a.tokens),
+                           a.out_stride, a.kv_head_limit, a.head_limit);
+      }
+    } else {
+      generations(first * heads, k_attention_vsa<kHmScales, kF16>);
+    }
+  }
+  a.cube0 = first;
+  a.q_blocks = all - first;
+  if (a.q_blocks > 0) generations(a.q_blocks * heads, k_attention_vsa<kHmScales, kF16>);
+  return hipGetLastError();
+}
+
 hipError_t launch_attention_vsa(const h3_attention_cfg& cfg, uint32_t token_count,
                                 uint32_t heads, const int32_t* qi, const float* qs,
                                 const int32_t* ki, const float* ks, const uint16_t* vt,
                                 uint16_t* out, const int32_t* routes, const int32_t* lengths,
-                                void* workspace, hipStream_t stream) {
+                                void* workspace, const VsaPrefix& prefix, hipStream_t stream) {
   Args a{};
   a.qi = qi;
   a.qs = qs;
@@ -1685,28 +1811,15 @@ hipError_t launch_attention_vsa(const h3_attention_cfg& cfg, uint32_t token_coun
                        dim3(256), 0, stream, ks, ks_hm, a.tokens, a.kv_head_limit);
     a.ks = ks_hm;
   }
-  // One launch per generation of resident workgroups (four per CU): its workgroups start
-  // together and walk their ascending key lists at about the same pace, so more of the tiles
-  // they share are still in L2 (measured at 129k tokens with token-major scales: 45.9 ms against
-  // 56.5 ms for one launch of all the work).
-  const uint32_t items = a.q_blocks * heads;
-  const uint32_t gen = std::max(1u, 4u * device_cus());
-  for (uint32_t base = 0; base < items; base += gen) {
-    a.base = base;
-    a.total = std::min(gen, items - base);
-    a.per_xcd = (a.total + 7) / 8;
-    if (workspace)
-      hipLaunchKernelGGL(k_attention_vsa<true>, dim3(a.per_xcd * 8), dim3(kVsaThreads), 0, stream, a);
-    else
-      hipLaunchKernelGGL(k_attention_vsa<false>, dim3(a.per_xcd * 8), dim3(kVsaThreads), 0, stream, a);
-  }
-  return hipGetLastError();
+  return workspace ? launch_vsa_cubes<true, false>(a, heads, prefix, stream)
+                   : launch_vsa_cubes<false, false>(a, heads, prefix, stream);
 }
 
 hipError_t launch_attention_vsa_f16(const h3_attention_cfg& cfg, uint32_t token_count,
                                     uint32_t heads, const uint16_t* q, const uint16_t* k,
                                     const uint16_t* v, uint16_t* out, const int32_t* routes,
-                                    const int32_t* lengths, hipStream_t stream) {
+                                    const int32_t* lengths, const VsaPrefix& prefix,
+                                    hipStream_t stream) {
   Args a{};
   a.qi = reinterpret_cast<const int32_t*>(q);
   a.ki = reinterpret_cast<const int32_t*>(k);
@@ -1727,17 +1840,7 @@ hipError_t launch_attention_vsa_f16(const h3_attention_cfg& cfg, uint32_t token_
   a.lengths = lengths;
   a.blocks = cfg.tokens / 64;
   a.scale = cfg.scale;
-  // Generations of resident workgroups as in launch_attention_vsa (four per CU).
-  const uint32_t items = a.q_blocks * heads;
-  const uint32_t gen = std::max(1u, 4u * device_cus());
-  for (uint32_t base = 0; base < items; base += gen) {
-    a.base = base;
-    a.total = std::min(gen, items - base);
-    a.per_xcd = (a.total + 7) / 8;
-    hipLaunchKernelGGL((k_attention_vsa<false, true>), dim3(a.per_xcd * 8), dim3(kVsaThreads), 0,
-                       stream, a);
-  }
-  return hipGetLastError();
+  return launch_vsa_cubes<false, true>(a, heads, prefix, stream);
 }
 
 }  // namespace h3

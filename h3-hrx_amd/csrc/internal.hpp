@@ -151,6 +151,16 @@ size_t scales_workspace_bytes(const h3_attention_cfg& cfg);
 hipError_t launch_attention_cross(const h3_cross_cfg& cfg, const int32_t* qi, const float* qs,
                                   const int32_t* ki, const float* ks, const uint16_t* vt,
                                   const uint8_t* key_mask, uint16_t* out, hipStream_t stream);
+// The query cubes [0, cubes) of every head whose routes keep (nearly) every key cube, the VSA
+// runtime's prefix: their own launches, each cube split into `splits` ranges of the key cubes when
+// `splits` > 1, with the ranges' partial results in `part` (vsa_part_bytes). Empty: no such cubes.
+struct VsaPrefix {
+  uint32_t cubes = 0, splits = 1;
+  float* part = nullptr;
+};
+// The number of ranges for `cubes` prefix cubes of `heads` heads over `blocks` key cubes, and the
+// bytes of their partial results (0 for one range).
+size_t vsa_part_bytes(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t* splits);
 // The int8 token-major attention over the cubes `routes` keeps (attention.hip). With a
 // `workspace` of scales_workspace_bytes(cfg) bytes the key scales are first transposed into it
 // (head-major) and the kernel reads them from there; with nullptr it reads the token-major
@@ -159,17 +169,23 @@ hipError_t launch_attention_vsa(const h3_attention_cfg& cfg, uint32_t token_coun
                                 uint32_t heads, const int32_t* qi, const float* qs,
                                 const int32_t* ki, const float* ks, const uint16_t* vt,
                                 uint16_t* out, const int32_t* routes, const int32_t* lengths,
-                                void* workspace, hipStream_t stream);
+                                void* workspace, const VsaPrefix& prefix, hipStream_t stream);
 // The f16 VSA attention (attention.hip): token-major f16 q, k, v; scores times cfg.scale.
 hipError_t launch_attention_vsa_f16(const h3_attention_cfg& cfg, uint32_t token_count,
                                     uint32_t heads, const uint16_t* q, const uint16_t* k,
                                     const uint16_t* v, uint16_t* out, const int32_t* routes,
-                                    const int32_t* lengths, hipStream_t stream);
+                                    const int32_t* lengths, const VsaPrefix& prefix,
+                                    hipStream_t stream);
 // h3_vsa_attention_i8 with a caller's workspace of at least scales_workspace_bytes(*cfg) bytes
 // (abi.cpp); with an empty view it reads the token-major scales as the public entry point does.
+// vsa_attention_f16: h3_vsa_attention_f16. Both with the runtime's prefix cubes.
+int vsa_attention_f16(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads, h3_view q,
+                      h3_view k, h3_view v, h3_view out, h3_view routes, h3_view lengths,
+                      const VsaPrefix& prefix, hipStream_t stream);
 int vsa_attention_i8_ws(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads,
                         h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt, h3_view out,
-                        h3_view routes, h3_view lengths, h3_view workspace, hipStream_t stream);
+                        h3_view routes, h3_view lengths, h3_view workspace,
+                        const VsaPrefix& prefix, hipStream_t stream);
 // h3_attention_i8qk_ws on the library's own static scratch array (noalloc.hip): the same
 // checks, except that the workspace, a device symbol's address, skips the runtime's pointer
 // query.

@@ -38,6 +38,8 @@ struct h3_vsa {
   h3_view q{}, k{}, v{}, qm{}, km{}, vm{}, coarse{}, scores{}, routes{}, out{};
   h3_view qi{}, ki{}, qs{}, ks{}, vt{}, zero{};
   h3_view ws{};  // the sparse attention's head-major copy of the key scales
+  h3::VsaPrefix prefix{};  // the prefix's query cubes, and the partial results of their key ranges
+  h3_view part{};
   std::vector<h3_view> means;  // the previous call's K mean of each layer
 };
 
@@ -48,7 +50,7 @@ namespace {
 void release(h3_vsa* r) {
   for (h3_view* v : {&r->src, &r->inverse, &r->lengths, &r->q, &r->k, &r->v, &r->qm, &r->km,
                      &r->vm, &r->coarse, &r->scores, &r->routes, &r->out, &r->qi, &r->ki, &r->qs,
-                     &r->ks, &r->vt, &r->zero, &r->ws})
+                     &r->ks, &r->vt, &r->zero, &r->ws, &r->part})
     if (v->ptr) (void)hipFree(v->ptr);
   for (h3_view& v : r->means)
     if (v.ptr) (void)hipFree(v.ptr);
@@ -252,6 +254,16 @@ int h3_vsa_build_bits(const int32_t* src, const int32_t* inverse, const int32_t*
       return st;
     }
   }
+  r->prefix.cubes = prefix_blocks;
+  const size_t part_bytes = vsa_part_bytes(heads, prefix_blocks, blocks, &r->prefix.splits);
+  if (part_bytes) {
+    if ((st = allocate(&r->part, part_bytes))) {
+      release(r);
+      delete r;
+      return st;
+    }
+    r->prefix.part = static_cast<float*>(r->part.ptr);
+  }
   if (bits == 16) {
     *out = r;
     set_error(H3_OK, "%s", "");
@@ -318,8 +330,9 @@ int h3_vsa_attend(h3_vsa* r, uint32_t layer, h3_view q, h3_view k, h3_view v, h3
     return st;
   if (r->bits == 16) {
     // 362-386: the f16 attention reads the gathered q, k, v as they are
-    if ((st = h3_vsa_attention_f16(&r->attention, c->padded, c->heads, r->q, r->k, r->v, r->out,
-                                   r->routes, r->lengths, stream)))
+    if ((st = vsa_attention_f16(&r->attention, c->padded, c->heads, r->q, r->k, r->v, r->out,
+                                r->routes, r->lengths, r->prefix,
+                                reinterpret_cast<hipStream_t>(stream))))
       return st;
   } else {
     // 290-333: INT8 operands (K centred on the layer's previous mean), V^T, sparse attention
@@ -330,7 +343,7 @@ int h3_vsa_attend(h3_vsa* r, uint32_t layer, h3_view q, h3_view k, h3_view v, h3
                         : h3_transpose_f16(&r->transpose, c->padded, c->padded, r->v, r->vt,
                                            stream)) ||
         (st = vsa_attention_i8_ws(&r->attention, c->padded, c->heads, r->qi, r->qs, r->ki, r->ks,
-                                  r->vt, r->out, r->routes, r->lengths, r->ws,
+                                  r->vt, r->out, r->routes, r->lengths, r->ws, r->prefix,
                                   reinterpret_cast<hipStream_t>(stream))))
       return st;
     // 334-346: this call's mean of the block K means, for the layer's next call
