@@ -332,19 +332,20 @@ void k_attention_split(Args g) {
 inline uint32_t div_up(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
 // The rule of split_plan prices a call in 64-key stages of k_attention_hm on a chip it does not
-// fill (1.5 us). Measured (S stages a block, s stages a unit):
-//   k_attention_hm      up to one round of blocks 8.5 + 1.5 S us (12.6 us at S = 3, 33.9 at 16, 57 at
-//                       32, 100 at 64); 1.12 times that for each full round of one block per CU (the
-//                       engine clock falls); after full rounds, a last round that fills a share f of
-//                       the CUs takes about (1 + f) / 2 of a full one (its blocks start as CUs free
-//                       up, and run at a higher clock)
-//   k_attention_split   6.7 + 4.2 s us a round of units (10 us at s = 1, 15.5-16.5 at 2, 22.5 at 4,
-//                       37-42 at 8): its operands come through each CU's L1 instead of being shared in
-//                       LDS, about 20 bytes a clock and CU
-// so 1,024 tokens of 8 heads take 15.5 us here against 33.9, 2,048 of 4 heads 22.6 against 56.5, and
-// 8,193 of 16 heads, whose last round would hold 16 blocks of one row each, 530 against 566; from
-// about 3,000 keys on a call that fills a quarter of the chip is faster undivided.
-constexpr float kMainFixed = 5.7f, kMainFull = 1.12f, kSplitStage = 2.8f, kSplitFixed = 4.5f;
+// fill (1.25 us). Measured inside Stack::attend, right after the operands' kernels (S stages a
+// block, s stages a unit):
+//   k_attention_hm      up to one round of blocks 6.4 + 1.25 S us (10.7 us at S = 3, 12.3 at 4, 15.8
+//                       at 7, 26.3 at 16); 1.34 times that for each full round of one block per CU
+//                       (the engine clock falls); after full rounds, a last round that fills a share
+//                       f of the CUs takes about (1 + f) / 2 of a full one (its blocks start as CUs
+//                       free up, and run at a higher clock)
+//   k_attention_split   9 + 4 s us a round of units (10.9-13.1 us at s = 1, 16.9 at 2): its operands
+//                       come through each CU's L1 instead of being shared in LDS, about 20 bytes a
+//                       clock and CU
+// so 1,024 tokens of 8 heads take 16.5 us here against 26.3, and 8,193 of 16 heads, whose last round
+// would hold 16 blocks of one row each, 530 against 566; calls of up to seven stages, and from about
+// 3,000 keys on those that fill a quarter of the chip, are faster undivided.
+constexpr float kMainFixed = 5.1f, kMainFull = 1.34f, kSplitStage = 3.2f, kSplitFixed = 7.2f;
 constexpr float kSecondLaunch = 2.0f;
 
 // Time of `blocks` blocks of `stages` stages on k_attention_hm.
@@ -375,8 +376,7 @@ SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t cu
   const uint32_t full = rows / kBlockQ, rest_tiles = div_up(rows % kBlockQ, kTileQ);
   const uint32_t full_blocks = full * heads, rest_blocks = rest_tiles ? heads : 0u;
   SplitPlan best{false, 0, 0, 0};
-  // a split has to gain more than the model's error: 2 %, and 1.5 us (118 keys of 2 heads, two
-  // stages, were 1.2 us slower divided)
+  // a split has to gain more than the model's error: 2 %, and a stage
   const float whole = main_time(full_blocks + rest_blocks, stages, cus);
   float best_time = std::min(0.98f * whole, whole - 1.0f);
   const uint32_t mains[2] = {full_blocks / cus * cus, full_blocks};
