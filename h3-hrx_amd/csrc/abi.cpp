@@ -135,9 +135,8 @@ int check_prepare_cfg(const char* stage, const h3_prepare_cfg* cfg, uint32_t tok
   return H3_OK;
 }
 
-int prepare_common(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens, h3_view x,
-                   h3_view mean, h3_view codes, h3_view scales, hipStream_t stream,
-                   bool head_major) {
+int check_prepare(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens, h3_view x,
+                  h3_view mean, h3_view codes, h3_view scales, bool head_major) {
   int st = check_prepare_cfg(stage, cfg, tokens, head_major);
   if (st) return st;
   const size_t rows_out = head_major ? (size_t)cfg->heads * cfg->token_capacity
@@ -147,7 +146,14 @@ int prepare_common(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens
                     rows_out * 128, rows_out * 4};
   if ((st = check_bindings(stage, views, need, 4))) return st;
   if ((st = check_aligned16(stage, {x, mean}))) return st;
-  if ((st = device_ready(stage))) return st;
+  return device_ready(stage);
+}
+
+int prepare_common(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens, h3_view x,
+                   h3_view mean, h3_view codes, h3_view scales, hipStream_t stream,
+                   bool head_major) {
+  const int st = check_prepare(stage, cfg, tokens, x, mean, codes, scales, head_major);
+  if (st) return st;
   return launched(stage, launch_prepare_qk(*cfg, tokens, head_major, x.ptr,
                                            static_cast<const float*>(mean.ptr),
                                            static_cast<int32_t*>(codes.ptr),
@@ -161,6 +167,19 @@ int rope_bindings(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens,
                     (size_t)tokens * 48 * 4};
   const int st = check_bindings(stage, views, need, 4);
   return st ? st : check_aligned16(stage, {x, weight, cos_t, sin_t});
+}
+
+int check_prepare_rope(const char* stage, const h3_prepare_cfg* cfg, uint32_t tokens, h3_view x,
+                       h3_view weight, h3_view cos_t, h3_view sin_t, h3_view codes,
+                       h3_view scales) {
+  int st = check_prepare_cfg(stage, cfg, tokens, true);
+  if (st) return st;
+  if ((st = rope_bindings(stage, cfg, tokens, x, weight, cos_t, sin_t))) return st;
+  const size_t rows_out = (size_t)cfg->heads * cfg->token_capacity;
+  h3_view views[2] = {codes, scales};
+  size_t need[2] = {rows_out * 128, rows_out * 4};
+  if ((st = check_bindings(stage, views, need, 2))) return st;
+  return device_ready(stage);
 }
 
 // Operand layouts of the attention kernels (attention.hip's modes).
@@ -350,8 +369,8 @@ int check_vsa_cfg(const char* stage, const h3_vsa_cfg* cfg) {
 }
 
 
-int transpose_common(const char* stage, const h3_transpose_cfg* cfg, uint32_t launch_rows,
-                     uint32_t rows, h3_view x, h3_view out, hipStream_t stream, bool qkv) {
+int check_transpose(const char* stage, const h3_transpose_cfg* cfg, uint32_t launch_rows,
+                    uint32_t rows, h3_view x, h3_view out, bool qkv) {
   if (!cfg) return set_error(H3_ERR_ARGUMENT, "%s: null config", stage);
   // kernels/transpose_f16.loom:7-9
   if (!in_range(cfg->width, 32, 65536, 32))
@@ -369,9 +388,15 @@ int transpose_common(const char* stage, const h3_transpose_cfg* cfg, uint32_t la
   const uint32_t stride = qkv ? 3 * cfg->width : cfg->width;
   h3_view views[2] = {x, out};
   size_t need[2] = {(size_t)rows * stride * 2, (size_t)cfg->width * cfg->row_capacity * 2};
-  int st = check_bindings(stage, views, need, 2);
+  const int st = check_bindings(stage, views, need, 2);
+  return st ? st : device_ready(stage);
+}
+
+int transpose_common(const char* stage, const h3_transpose_cfg* cfg, uint32_t launch_rows,
+                     uint32_t rows, h3_view x, h3_view out, hipStream_t stream, bool qkv) {
+  const int st = check_transpose(stage, cfg, launch_rows, rows, x, out, qkv);
   if (st) return st;
-  if ((st = device_ready(stage))) return st;
+  const uint32_t stride = qkv ? 3 * cfg->width : cfg->width;
   const uint32_t tile = (qkv && cfg->width % 64 == 0) ? 64 : 32;
   return launched(stage, launch_transpose(cfg->width, cfg->row_capacity, stride,
                                           qkv ? 2 * cfg->width : 0, cfg->elem, tile, launch_rows,
@@ -379,6 +404,45 @@ int transpose_common(const char* stage, const h3_transpose_cfg* cfg, uint32_t la
 }
 
 }  // namespace
+
+int prepare_separate(const h3_prepare_cfg* pq, const h3_prepare_cfg* pk,
+                     const h3_transpose_cfg* t, bool head_major, uint32_t tokens, h3_view q,
+                     h3_view k, h3_view v, h3_view kmean, h3_view qi, h3_view qs, h3_view ki,
+                     h3_view ks, h3_view vt, h3_stream stream) {
+  const char* stage = head_major ? "prepare_qk_i8hm" : "prepare_qk_i8";
+  int st;
+  if ((st = check_prepare(stage, pq, tokens, q, {}, qi, qs, head_major)) ||
+      (st = check_prepare(stage, pk, tokens, k, kmean, ki, ks, head_major)) ||
+      (st = check_transpose("transpose_f16", t, t->row_capacity, tokens, v, vt, false)))
+    return st;
+  return launched(stage, launch_prepare_separate(
+                             *pq, *pk, *t, tokens, head_major, t->row_capacity, q.ptr, k.ptr,
+                             v.ptr, static_cast<const float*>(kmean.ptr),
+                             static_cast<int32_t*>(qi.ptr), static_cast<float*>(qs.ptr),
+                             static_cast<int32_t*>(ki.ptr), static_cast<float*>(ks.ptr),
+                             static_cast<uint16_t*>(vt.ptr),
+                             reinterpret_cast<hipStream_t>(stream)));
+}
+
+int prepare_fused(const h3_prepare_cfg* pq, const h3_prepare_cfg* pk, const h3_transpose_cfg* t,
+                  uint32_t tokens, h3_view x, h3_view qnorm, h3_view knorm, h3_view cos_t,
+                  h3_view sin_t, h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt,
+                  h3_stream stream) {
+  const char* stage = "prepare_qk_rope_i8hm";
+  int st;
+  if ((st = check_prepare_rope(stage, pq, tokens, x, qnorm, cos_t, sin_t, qi, qs)) ||
+      (st = check_prepare_rope(stage, pk, tokens, x, knorm, cos_t, sin_t, ki, ks)) ||
+      (st = check_transpose("transpose_qkv_v_f16", t, tokens, tokens, x, vt, true)))
+    return st;
+  return launched(stage, launch_prepare_fused(
+                             *pq, *pk, *t, tokens, x.ptr, static_cast<const float*>(qnorm.ptr),
+                             static_cast<const float*>(knorm.ptr),
+                             static_cast<const float*>(cos_t.ptr),
+                             static_cast<const float*>(sin_t.ptr), static_cast<int32_t*>(qi.ptr),
+                             static_cast<float*>(qs.ptr), static_cast<int32_t*>(ki.ptr),
+                             static_cast<float*>(ks.ptr), static_cast<uint16_t*>(vt.ptr),
+                             reinterpret_cast<hipStream_t>(stream)));
+}
 
 int attention_i8qk_static_ws(const h3_attention_cfg* cfg, uint32_t token_count, uint32_t heads,
                              h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt,
@@ -516,14 +580,8 @@ int h3_prepare_qk_rope_i8hm(const h3_prepare_cfg* cfg, uint32_t tokens, h3_view 
                             h3_view weight, h3_view cos_t, h3_view sin_t, h3_view codes,
                             h3_view scales, h3_stream stream) {
   const char* stage = "prepare_qk_rope_i8hm";
-  int st = check_prepare_cfg(stage, cfg, tokens, true);
+  const int st = check_prepare_rope(stage, cfg, tokens, x, weight, cos_t, sin_t, codes, scales);
   if (st) return st;
-  if ((st = rope_bindings(stage, cfg, tokens, x, weight, cos_t, sin_t))) return st;
-  const size_t rows_out = (size_t)cfg->heads * cfg->token_capacity;
-  h3_view views[2] = {codes, scales};
-  size_t need[2] = {rows_out * 128, rows_out * 4};
-  if ((st = check_bindings(stage, views, need, 2))) return st;
-  if ((st = device_ready(stage))) return st;
   return launched(stage, launch_prepare_qk_rope(
                              *cfg, tokens, x.ptr, static_cast<const float*>(weight.ptr),
                              static_cast<const float*>(cos_t.ptr),

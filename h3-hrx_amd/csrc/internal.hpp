@@ -49,6 +49,31 @@ hipError_t launch_prepare_qk_i4(const h3_prepare_cfg& cfg, uint32_t tokens, cons
 hipError_t launch_prepare_qk_rope(const h3_prepare_cfg& cfg, uint32_t tokens, const void* x,
                                   const float* weight, const float* cos_t, const float* sin_t,
                                   int32_t* codes, float* scales, hipStream_t stream);
+// Stack::attend's preparations in one launch: the quantizer of Q (zero mean) and of K (less `kmean`
+// unless null) from separate rows, and V^T over ceil(launch_rows / 32) column tiles.
+hipError_t launch_prepare_separate(const h3_prepare_cfg& q, const h3_prepare_cfg& k,
+                                   const h3_transpose_cfg& t, uint32_t tokens, int head_major,
+                                   uint32_t launch_rows, const void* xq, const void* xk,
+                                   const void* xv, const float* kmean, int32_t* qi, float* qs,
+                                   int32_t* ki, float* ks, uint16_t* vt, hipStream_t stream);
+// Stack::attend_fused's preparations without smoothing in one launch, from the fused QKV rows `x`:
+// the RoPE quantizer of Q and of K and V^T.
+hipError_t launch_prepare_fused(const h3_prepare_cfg& q, const h3_prepare_cfg& k,
+                                const h3_transpose_cfg& t, uint32_t tokens, const void* x,
+                                const float* qweight, const float* kweight, const float* cos_t,
+                                const float* sin_t, int32_t* qi, float* qs, int32_t* ki, float* ks,
+                                uint16_t* vt, hipStream_t stream);
+// The operands of a Stack call through one launch, with the checks of the entries it stands for
+// (h3_prepare_qk_i8 or _i8hm of q and k, h3_transpose_f16; h3_prepare_qk_rope_i8hm of q and k,
+// h3_transpose_qkv_v_f16), all before the launch (abi.cpp). kmean: an empty view for no smoothing.
+int prepare_separate(const h3_prepare_cfg* pq, const h3_prepare_cfg* pk,
+                     const h3_transpose_cfg* t, bool head_major, uint32_t tokens, h3_view q,
+                     h3_view k, h3_view v, h3_view kmean, h3_view qi, h3_view qs, h3_view ki,
+                     h3_view ks, h3_view vt, h3_stream stream);
+int prepare_fused(const h3_prepare_cfg* pq, const h3_prepare_cfg* pk, const h3_transpose_cfg* t,
+                  uint32_t tokens, h3_view x, h3_view qnorm, h3_view knorm, h3_view cos_t,
+                  h3_view sin_t, h3_view qi, h3_view qs, h3_view ki, h3_view ks, h3_view vt,
+                  h3_stream stream);
 hipError_t launch_rope_qknorm(const h3_rope_cfg& cfg, uint32_t tokens, const void* x,
                               const float* qweight, const float* kweight, const float* cos_t,
                               const float* sin_t, uint16_t* q_out, uint16_t* k_out,

@@ -369,25 +369,24 @@ __device__ __forceinline__ uint2 quantize_row16_i4(const float (&r)[16], float e
 
 // (token, head) rows (kernels/prepare_qk_i8.loom, prepare_qk_i8hm.loom; with kI4 the token-major
 // int4 operands of kernels/prepare_qk_i4.loom, codes [tokens][heads*16] i32), one per 8-lane
-// group; group g of block b takes rows b*32*kRowsAhead + 32i + g, i < kRowsAhead, all loads
+// group; group g of block b takes rows b*32*kAhead + 32i + g, i < kAhead, all loads
 // issued before the first row is processed. Head-major rows walk tokens fastest (contiguous code
 // stores), token-major rows walk heads.
-template <bool kHeadMajor, int kElem, bool kMean, bool kI4 = false>
-__global__ __launch_bounds__(256) void k_prepare_qk(const void* __restrict__ x,
-                                                    const float* __restrict__ mean,
-                                                    int32_t* __restrict__ codes,
-                                                    float* __restrict__ scales, uint32_t tokens,
-                                                    uint32_t row_stride, uint32_t head_offset,
-                                                    uint32_t heads, uint32_t capacity,
-                                                    float extra) {
+template <bool kHeadMajor, int kElem, bool kMean, bool kI4, int kAhead>
+__device__ __forceinline__ void prepare_rows(uint32_t block, const void* __restrict__ x,
+                                             const float* __restrict__ mean,
+                                             int32_t* __restrict__ codes,
+                                             float* __restrict__ scales, uint32_t tokens,
+                                             uint32_t row_stride, uint32_t head_offset,
+                                             uint32_t heads, uint32_t capacity, float extra) {
   const int lane = threadIdx.x & 63;
   const int l = local8(lane);
   const uint32_t first =
-      blockIdx.x * kRopeGroups * kRowsAhead + 8 * (threadIdx.x >> 6) + group8(lane);
+      block * kRopeGroups * kAhead + 8 * (threadIdx.x >> 6) + group8(lane);
   const uint32_t total = tokens * heads;
-  uint4 in[kRowsAhead][2];
+  uint4 in[kAhead][2];
 #pragma unroll
-  for (int i = 0; i < kRowsAhead; ++i) {
+  for (int i = 0; i < kAhead; ++i) {
     const uint32_t row = first + kRopeGroups * i;
     if (row >= total) break;
     const uint32_t t = kHeadMajor ? row % tokens : row / heads;
@@ -397,7 +396,7 @@ __global__ __launch_bounds__(256) void k_prepare_qk(const void* __restrict__ x,
     in[i][1] = load8(x, at + 8);
   }
 #pragma unroll
-  for (int i = 0; i < kRowsAhead; ++i) {
+  for (int i = 0; i < kAhead; ++i) {
     const uint32_t row = first + kRopeGroups * i;
     if (row >= total) break;
     const uint32_t t = kHeadMajor ? row % tokens : row / heads;
@@ -436,21 +435,35 @@ __global__ __launch_bounds__(256) void k_prepare_qk(const void* __restrict__ x,
   }
 }
 
+template <bool kHeadMajor, int kElem, bool kMean, bool kI4 = false>
+__global__ __launch_bounds__(256) void k_prepare_qk(const void* __restrict__ x,
+                                                    const float* __restrict__ mean,
+                                                    int32_t* __restrict__ codes,
+                                                    float* __restrict__ scales, uint32_t tokens,
+                                                    uint32_t row_stride, uint32_t head_offset,
+                                                    uint32_t heads, uint32_t capacity,
+                                                    float extra) {
+  prepare_rows<kHeadMajor, kElem, kMean, kI4, kRowsAhead>(blockIdx.x, x, mean, codes, scales,
+                                                          tokens, row_stride, head_offset, heads,
+                                                          capacity, extra);
+}
+
 // RMSNorm + RoPE + f16 rounding + (optional mean subtraction) + quantizer, head-major output
 // (kernels/prepare_qk_rope_i8hm.loom:94-239; mean == nullptr is the reference's unsmoothed
 // kernel, a mean is this build's fused K-smoothing second pass). One 8-lane group owns one token
 // and walks its heads with kRowsAhead heads in flight: the token's RoPE tables are read once
 // (not once per head), its heads' inputs are one contiguous run of the fused row, and the 32
 // groups of a workgroup write 32 consecutive head-major rows (4 KiB) per head. Group g of wave w
-// takes token 32 * block + 8w + g.
+// takes token 32 * block + 8w + g, heads head0 .. heads - 1.
 template <int kElem, bool kMean>
-__global__ __launch_bounds__(256) void k_prepare_qk_rope(
-    const void* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, const float* __restrict__ mean, int32_t* __restrict__ codes,
-    float* __restrict__ scales, uint32_t tokens, uint32_t row_stride, uint32_t head_offset,
-    uint32_t heads, uint32_t capacity, float extra, float eps) {
+__device__ __forceinline__ void prepare_rope_rows(
+    uint32_t block, const void* __restrict__ x, const float* __restrict__ weight,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    const float* __restrict__ mean, int32_t* __restrict__ codes, float* __restrict__ scales,
+    uint32_t tokens, uint32_t row_stride, uint32_t head_offset, uint32_t head0, uint32_t heads,
+    uint32_t capacity, float extra, float eps) {
   const int lane = threadIdx.x & 63;
-  const uint32_t t = blockIdx.x * kRopeGroups + 8 * (threadIdx.x >> 6) + group8(lane);
+  const uint32_t t = block * kRopeGroups + 8 * (threadIdx.x >> 6) + group8(lane);
   const int l = local8(lane);
   if (t >= tokens) return;
   const RopeLane16 tab = rope_lane16(l, weight, cos_t + (size_t)t * 48, sin_t + (size_t)t * 48);
@@ -458,11 +471,11 @@ __global__ __launch_bounds__(256) void k_prepare_qk_rope(
   uint4 ring[kRowsAhead][2];  // heads h .. h + kRowsAhead - 1 in flight
 #pragma unroll
   for (int i = 0; i < kRowsAhead; ++i)
-    if ((uint32_t)i < heads) {
-      ring[i][0] = load8(x, row0 + 128u * i);
-      ring[i][1] = load8(x, row0 + 128u * i + 8);
+    if (head0 + i < heads) {
+      ring[i][0] = load8(x, row0 + 128u * (head0 + i));
+      ring[i][1] = load8(x, row0 + 128u * (head0 + i) + 8);
     }
-  for (uint32_t h0 = 0; h0 < heads; h0 += kRowsAhead) {
+  for (uint32_t h0 = head0; h0 < heads; h0 += kRowsAhead) {
 #pragma unroll
     for (int i = 0; i < kRowsAhead; ++i) {
       const uint32_t h = h0 + i;
@@ -508,6 +521,21 @@ __global__ __launch_bounds__(256) void k_prepare_qk_rope(
   }
 }
 
+// Workgroup b of a launch over `token_blocks` x ceil(heads / chunk) takes 32 tokens and `chunk`
+// heads. A chunk costs its tokens' tables and norm weights once more, so a launch is cut in chunks
+// only as far as it takes to fill the chip (rope_chunk).
+template <int kElem, bool kMean>
+__global__ __launch_bounds__(256) void k_prepare_qk_rope(
+    const void* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, const float* __restrict__ mean, int32_t* __restrict__ codes,
+    float* __restrict__ scales, uint32_t tokens, uint32_t row_stride, uint32_t head_offset,
+    uint32_t heads, uint32_t capacity, float extra, float eps, uint32_t chunk) {
+  const uint32_t head0 = blockIdx.y * chunk;
+  prepare_rope_rows<kElem, kMean>(blockIdx.x, x, weight, cos_t, sin_t, mean, codes, scales, tokens,
+                                  row_stride, head_offset, head0, min(heads, head0 + chunk),
+                                  capacity, extra, eps);
+}
+
 // RMSNorm + RoPE of Q and K heads to f16, V optionally copied (kernels/rope_qknorm_f16.loom).
 // Rows are (token, head) over heads + kv_heads (+ kv_heads copy rows).
 __global__ __launch_bounds__(256) void k_rope_qknorm(
@@ -548,7 +576,8 @@ __global__ __launch_bounds__(256) void k_rope_qknorm(
 // ---------------------------------------------------------------- column means
 
 // mean[c] = (sum_t x[t][c]) / tokens, one lane per column summing tokens in order
-// (kernels/colmean_f32.loom in-file 30-40). Eight loads are issued ahead of the dependent adds.
+// (kernels/colmean_f32.loom in-file 30-40), 16 loads issued ahead of the dependent adds: for few
+// tokens, and inputs that are not 16-byte aligned. The others take k_rope_colmean<false>.
 __global__ __launch_bounds__(64) void k_colmean(const void* __restrict__ x,
                                                 float* __restrict__ mean, uint32_t tokens,
                                                 uint32_t width, uint32_t row_stride,
@@ -639,6 +668,7 @@ struct PairToken {  // the raw inputs of one token for a workgroup's 16 channels
   float r;
 };
 
+template <bool kRope>
 __device__ __forceinline__ void load_pair_token(PairToken& in, const void* x, const float* r_in,
                                                 const float* cos_t, const float* sin_t,
                                                 uint32_t t, uint32_t tokens, size_t col_a,
@@ -648,6 +678,7 @@ __device__ __forceinline__ void load_pair_token(PairToken& in, const void* x, co
   const uint16_t* row = reinterpret_cast<const uint16_t*>(x) + (size_t)t * row_stride;
   in.a = *reinterpret_cast<const uint4*>(row + col_a);
   in.b = *reinterpret_cast<const uint4*>(row + col_b);
+  if constexpr (!kRope) return;
   in.r = r_in[r_base + t];
   if (rotated) {
     const float* ct = cos_t + (size_t)t * 48 + tab0;
@@ -668,6 +699,11 @@ __device__ __forceinline__ void unpack8(uint4 b, uint32_t elem, float (&v)[8]) {
   }
 }
 
+// kRope false: the column mean of x itself (h3_colmean_f32), 16 adjacent columns per workgroup; the
+// producers only widen, and weight, the tables and r_in are not read. One lane per column with 16
+// loads in flight was bound by their latency, 34 ns a row against the chain's 3.54: 86 -> 26 us at
+// 2,501 x 7,168, 5,660 -> 730 us at 129,024 x 4,096.
+template <bool kRope>
 __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
     const void* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const float* __restrict__ r_in, float* __restrict__ mean,
@@ -678,9 +714,9 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
   const uint32_t logical = (b % 8) * per_xcd + b / 8;  // workgroup b runs on XCD b % 8
   if (logical >= total) return;                       // whole workgroup, before any barrier
   const uint32_t h = logical / kSlabs, k = logical % kSlabs;
-  const bool rotated = k < 6;
+  const bool rotated = kRope && k < 6;
   // channels of tile rows 0-7 and 8-15
-  const uint32_t ca = rotated ? 8 * k : 96 + 16 * (k - 6);
+  const uint32_t ca = !kRope ? 16 * k : rotated ? 8 * k : 96 + 16 * (k - 6);
   const uint32_t cb = rotated ? ca + 48 : ca + 8;
   const size_t col_a = head_offset + 128u * h + ca, col_b = head_offset + 128u * h + cb;
   const size_t r_base = (size_t)h * capacity;
@@ -692,8 +728,8 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
   float wa[8], wb[8];
   PairToken ring[kRing];
   auto load = [&](PairToken& in, uint32_t j) {
-    load_pair_token(in, x, r_in, cos_t, sin_t, j * kChunk + p, tokens, col_a, col_b, row_stride,
-                    r_base, 8 * k, rotated);
+    load_pair_token<kRope>(in, x, r_in, cos_t, sin_t, j * kChunk + p, tokens, col_a, col_b,
+                           row_stride, r_base, 8 * k, rotated);
   };
   // Chunk j's values into tile buffer j % 2: the operations of rmsnorm_rope_f16, channel by
   // channel (rope_channel), so the values are bit-identical to h3_rope_qknorm_f16's output.
@@ -703,7 +739,13 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
     float va[8], vb[8];
     unpack8(in.a, elem, va);
     unpack8(in.b, elem, vb);
-    if (rotated) {
+    if constexpr (!kRope) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        dst[i][p] = va[i];
+        dst[8 + i][p] = vb[i];
+      }
+    } else if (rotated) {
       const float cc[8] = {in.c[0].x, in.c[0].y, in.c[0].z, in.c[0].w,
                            in.c[1].x, in.c[1].y, in.c[1].z, in.c[1].w};
       const float ss[8] = {in.s[0].x, in.s[0].y, in.s[0].z, in.s[0].w,
@@ -723,10 +765,12 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
   };
 
   if (producer) {
+    if constexpr (kRope) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      wa[i] = weight[ca + i];
-      wb[i] = weight[cb + i];
+      for (int i = 0; i < 8; ++i) {
+        wa[i] = weight[ca + i];
+        wb[i] = weight[cb + i];
+      }
     }
 #pragma unroll
     for (int i = 0; i < kRing; ++i)
@@ -748,12 +792,13 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
     if (threadIdx.x < kSlab) {
       const float* col = tile[j & 1][lane];
       const uint32_t n = min((uint32_t)kChunk, tokens - j * kChunk);
-      if (n == kChunk) {
+      const uint32_t groups = n / 32;
+      if (groups > 0) {
         float4 cur[8], nxt[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) cur[i] = *reinterpret_cast<const float4*>(col + 4 * i);
-        for (int g = 0; g < kChunk / 32; ++g) {
-          if (g + 1 < kChunk / 32) {
+        for (uint32_t g = 0; g < groups; ++g) {
+          if (g + 1 < groups) {
 #pragma unroll
             for (int i = 0; i < 8; ++i)
               nxt[i] = *reinterpret_cast<const float4*>(col + 32 * (g + 1) + 4 * i);
@@ -768,9 +813,8 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
 #pragma unroll
           for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
         }
-      } else {
-        for (uint32_t i = 0; i < n; ++i) acc = acc + col[i];
       }
+      for (uint32_t i = 32 * groups; i < n; ++i) acc = acc + col[i];
     }
     __syncthreads();
   };
@@ -796,17 +840,17 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
 // kGather: row r of the input is row src[r] of x (a zero row where src[r] >= src_rows), and each
 // loaded piece is also written, as loaded, to gathered[r][c] (the VSA runtime's gathered v,
 // [rows][width], and its V^T from one read of x).
+typedef uint16_t TransposeTile[64][64 + 2];
 template <bool kGather>
-__global__ __launch_bounds__(256) void k_transpose(const uint16_t* __restrict__ x,
-                                                   uint16_t* __restrict__ out, uint32_t rows,
-                                                   uint32_t clear_to, uint32_t width,
-                                                   uint32_t capacity, uint32_t row_stride,
-                                                   uint32_t col_offset, uint32_t elem,
-                                                   const int32_t* __restrict__ src,
-                                                   uint32_t src_rows,
-                                                   uint16_t* __restrict__ gathered) {
-  __shared__ uint16_t tile[64][64 + 2];
-  const uint32_t c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
+__device__ __forceinline__ void transpose_tile(TransposeTile& tile, uint32_t c0, uint32_t r0,
+                                               const uint16_t* __restrict__ x,
+                                               uint16_t* __restrict__ out, uint32_t rows,
+                                               uint32_t clear_to, uint32_t width,
+                                               uint32_t capacity, uint32_t row_stride,
+                                               uint32_t col_offset, uint32_t elem,
+                                               const int32_t* __restrict__ src,
+                                               uint32_t src_rows,
+                                               uint16_t* __restrict__ gathered) {
   // load: 64 rows x 64 columns, lane -> row i/16 (+16k), columns 4*(i%16)..+3
   const int lr = threadIdx.x >> 4, lc = (threadIdx.x & 15) * 4;
 #pragma unroll
@@ -860,9 +904,199 @@ __global__ __launch_bounds__(256) void k_transpose(const uint16_t* __restrict__ 
   }
 }
 
+template <bool kGather>
+__global__ __launch_bounds__(256) void k_transpose(const uint16_t* __restrict__ x,
+                                                   uint16_t* __restrict__ out, uint32_t rows,
+                                                   uint32_t clear_to, uint32_t width,
+                                                   uint32_t capacity, uint32_t row_stride,
+                                                   uint32_t col_offset, uint32_t elem,
+                                                   const int32_t* __restrict__ src,
+                                                   uint32_t src_rows,
+                                                   uint16_t* __restrict__ gathered) {
+  __shared__ TransposeTile tile;
+  transpose_tile<kGather>(tile, blockIdx.x * 64, blockIdx.y * 64, x, out, rows, clear_to, width,
+                          capacity, row_stride, col_offset, elem, src, src_rows, gathered);
+}
+
+// ---------------------------------------------------------------- the operands of one call
+
+// Stack::attend's three preparations as one launch: workgroups [0, rows) quantize Q rows, [rows,
+// 2 rows) K rows (less `kmean`, if any), the others transpose V in 64 x 64 tiles. The three are
+// independent and each small: at 129 tokens x 56 heads the separate launches took 5.5 + 5.5 + 3.4 us
+// on the GPU and three launches' time on the host. kAhead: rows in flight per 8-lane group
+// (prepare_rows); 1 where 4 would leave the chip less than a workgroup per CU and operand.
+struct SeparateArgs {
+  const void *q, *k, *v;
+  const float* kmean;
+  int32_t *qi, *ki;
+  float *qs, *ks;
+  uint16_t* vt;
+  uint32_t tokens, width, heads, capacity;
+  float extra_q, extra_k;
+  uint32_t rows;           // workgroups per operand
+  uint32_t tiles_x;        // V^T: 64-column tiles of the width
+  uint32_t clear_to, row_capacity;
+};
+template <bool kHeadMajor, int kElem, bool kMean, int kAhead>
+__global__ __launch_bounds__(256) void k_prepare_separate(SeparateArgs a) {
+  __shared__ TransposeTile tile;
+  const uint32_t b = blockIdx.x;
+  if (b < a.rows) {
+    prepare_rows<kHeadMajor, kElem, false, false, kAhead>(b, a.q, nullptr, a.qi, a.qs, a.tokens,
+                                                          a.width, 0, a.heads, a.capacity,
+                                                          a.extra_q);
+  } else if (b < 2 * a.rows) {
+    prepare_rows<kHeadMajor, kElem, kMean, false, kAhead>(b - a.rows, a.k, a.kmean, a.ki, a.ks,
+                                                          a.tokens, a.width, 0, a.heads,
+                                                          a.capacity, a.extra_k);
+  } else {
+    const uint32_t t = b - 2 * a.rows;
+    transpose_tile<false>(tile, t % a.tiles_x * 64, t / a.tiles_x * 64,
+                          static_cast<const uint16_t*>(a.v), a.vt, a.tokens, a.clear_to, a.width,
+                          a.row_capacity, a.width, 0, kElem, nullptr, 0u, nullptr);
+  }
+}
+
+// Stack::attend_fused's three preparations (without smoothing) as one launch, from the fused QKV
+// rows: workgroups [0, rows) the RoPE quantizer of Q, [rows, 2 rows) of K (each `token_blocks` x
+// head chunks), the others V^T.
+struct FusedArgs {
+  const void* x;
+  const float *qweight, *kweight, *cos_t, *sin_t;
+  int32_t *qi, *ki;
+  float *qs, *ks;
+  uint16_t* vt;
+  uint32_t tokens, row_stride, heads, capacity, k_offset;
+  float extra_q, extra_k, eps;
+  uint32_t rows, token_blocks, chunk;
+  uint32_t tiles_x, width, clear_to, row_capacity;
+};
+template <int kElem>
+__global__ __launch_bounds__(256) void k_prepare_fused(FusedArgs a) {
+  __shared__ TransposeTile tile;
+  const uint32_t b = blockIdx.x;
+  if (b < 2 * a.rows) {
+    const bool is_q = b < a.rows;
+    const uint32_t u = is_q ? b : b - a.rows;
+    const uint32_t head0 = u / a.token_blocks * a.chunk;
+    prepare_rope_rows<kElem, false>(u % a.token_blocks, a.x, is_q ? a.qweight : a.kweight, a.cos_t,
+                                    a.sin_t, nullptr, is_q ? a.qi : a.ki, is_q ? a.qs : a.ks,
+                                    a.tokens, a.row_stride, is_q ? 0u : a.k_offset, head0,
+                                    min(a.heads, head0 + a.chunk), a.capacity,
+                                    is_q ? a.extra_q : a.extra_k, a.eps);
+  } else {
+    const uint32_t t = b - 2 * a.rows;
+    transpose_tile<false>(tile, t % a.tiles_x * 64, t / a.tiles_x * 64,
+                          static_cast<const uint16_t*>(a.x), a.vt, a.tokens, a.clear_to, a.width,
+                          a.row_capacity, a.row_stride, 2 * a.width, kElem, nullptr, 0u, nullptr);
+  }
+}
+
 inline uint32_t div_up(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
+// Heads per workgroup of the RoPE quantizer. One workgroup per 32 tokens walking all heads leaves a
+// short sequence's launch with few workgroups and a long serial walk: at 4,097 tokens x 56 heads (129
+// workgroups) 74 us, in chunks of 8 heads 33 us; 8,193 x 16 34 -> 23 (chunks of 4); 31,104 x 32 116 ->
+// 109. From 65,536 tokens on whole walks are as fast (129,024 x 32: 417 against 420 us) and read the
+// tables once.
+uint32_t rope_chunk(uint32_t tokens, uint32_t heads) {
+  const uint32_t blocks = div_up(tokens, kRopeGroups);
+  if (blocks >= 8 * device_cus()) return div_up(heads, kRowsAhead) * kRowsAhead;
+  return blocks * div_up(heads, 8) < 4 * device_cus() ? 4 : 8;
+}
+
 }  // namespace
+
+hipError_t launch_prepare_separate(const h3_prepare_cfg& q, const h3_prepare_cfg& k,
+                                   const h3_transpose_cfg& t, uint32_t tokens, int head_major,
+                                   uint32_t launch_rows, const void* xq, const void* xk,
+                                   const void* xv, const float* kmean, int32_t* qi, float* qs,
+                                   int32_t* ki, float* ks, uint16_t* vt, hipStream_t stream) {
+  SeparateArgs a{};
+  a.q = xq;
+  a.k = xk;
+  a.v = xv;
+  a.kmean = kmean;
+  a.qi = qi;
+  a.ki = ki;
+  a.qs = qs;
+  a.ks = ks;
+  a.vt = vt;
+  a.tokens = tokens;
+  a.width = q.row_stride;
+  a.heads = q.heads;
+  a.capacity = head_major ? q.token_capacity : 0u;
+  a.extra_q = q.extra_scale;
+  a.extra_k = k.extra_scale;
+  a.row_capacity = t.row_capacity;
+  a.clear_to = std::min(div_up(launch_rows, 32) * 32, t.row_capacity);
+  a.tiles_x = div_up(t.width, 64);
+  const uint32_t total = tokens * q.heads;
+  const bool one = div_up(total, kRopeGroups * kRowsAhead) < device_cus();
+  a.rows = div_up(total, kRopeGroups * (one ? 1 : kRowsAhead));
+  const dim3 grid(2 * a.rows + a.tiles_x * div_up(a.clear_to, 64));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
+  };
+  auto pick = [&](auto hm, auto elem) {
+    constexpr bool kHm = decltype(hm)::value;
+    constexpr int kElem = decltype(elem)::value;
+    if (kmean)
+      one ? launch(k_prepare_separate<kHm, kElem, true, 1>)
+          : launch(k_prepare_separate<kHm, kElem, true, kRowsAhead>);
+    else
+      one ? launch(k_prepare_separate<kHm, kElem, false, 1>)
+          : launch(k_prepare_separate<kHm, kElem, false, kRowsAhead>);
+  };
+  const bool bf16 = q.elem == H3_ELEM_BF16;
+  using F16 = std::integral_constant<int, H3_ELEM_F16>;
+  using BF16 = std::integral_constant<int, H3_ELEM_BF16>;
+  if (head_major)
+    bf16 ? pick(std::true_type{}, BF16{}) : pick(std::true_type{}, F16{});
+  else
+    bf16 ? pick(std::false_type{}, BF16{}) : pick(std::false_type{}, F16{});
+  return hipGetLastError();
+}
+
+hipError_t launch_prepare_fused(const h3_prepare_cfg& q, const h3_prepare_cfg& k,
+                                const h3_transpose_cfg& t, uint32_t tokens, const void* x,
+                                const float* qweight, const float* kweight, const float* cos_t,
+                                const float* sin_t, int32_t* qi, float* qs, int32_t* ki, float* ks,
+                                uint16_t* vt, hipStream_t stream) {
+  FusedArgs a{};
+  a.x = x;
+  a.qweight = qweight;
+  a.kweight = kweight;
+  a.cos_t = cos_t;
+  a.sin_t = sin_t;
+  a.qi = qi;
+  a.ki = ki;
+  a.qs = qs;
+  a.ks = ks;
+  a.vt = vt;
+  a.tokens = tokens;
+  a.row_stride = q.row_stride;
+  a.heads = q.heads;
+  a.capacity = q.token_capacity;
+  a.k_offset = k.head_offset;
+  a.extra_q = q.extra_scale;
+  a.extra_k = k.extra_scale;
+  a.eps = q.eps;
+  a.chunk = rope_chunk(tokens, q.heads);
+  a.token_blocks = div_up(tokens, kRopeGroups);
+  a.rows = a.token_blocks * div_up(q.heads, a.chunk);
+  a.width = t.width;
+  a.row_capacity = t.row_capacity;
+  const uint32_t tile = t.width % 64 == 0 ? 64 : 32;  // h3_transpose_qkv_v_f16's column tiles
+  a.clear_to = std::min(div_up(tokens, tile) * tile, t.row_capacity);
+  a.tiles_x = div_up(t.width, 64);
+  const dim3 grid(2 * a.rows + a.tiles_x * div_up(a.clear_to, 64));
+  if (q.elem == H3_ELEM_BF16)
+    hipLaunchKernelGGL(k_prepare_fused<H3_ELEM_BF16>, grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL(k_prepare_fused<H3_ELEM_F16>, grid, dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_prepare_qk(const h3_prepare_cfg& cfg, uint32_t tokens, int head_major,
                              const void* x, const float* mean, int32_t* codes, float* scales,
@@ -919,11 +1153,12 @@ hipError_t launch_prepare_qk_rope_mean(const h3_prepare_cfg& cfg, uint32_t token
                                        const float* weight, const float* cos_t,
                                        const float* sin_t, const float* mean, int32_t* codes,
                                        float* scales, hipStream_t stream) {
-  const dim3 grid(div_up(tokens, kRopeGroups));
+  const uint32_t chunk = rope_chunk(tokens, cfg.heads);
+  const dim3 grid(div_up(tokens, kRopeGroups), div_up(cfg.heads, chunk));
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, weight, cos_t, sin_t, mean, codes,
                        scales, tokens, cfg.row_stride, cfg.head_offset, cfg.heads,
-                       cfg.token_capacity, cfg.extra_scale, cfg.eps);
+                       cfg.token_capacity, cfg.extra_scale, cfg.eps, chunk);
   };
   const bool bf16 = cfg.elem == H3_ELEM_BF16;
   if (mean)
@@ -947,6 +1182,16 @@ hipError_t launch_rope_qknorm(const h3_rope_cfg& cfg, uint32_t tokens, const voi
 
 hipError_t launch_colmean(uint32_t width, uint32_t row_stride, uint32_t elem, uint32_t tokens,
                           const void* x, float* mean, hipStream_t stream) {
+  // 16-byte loads; up to about 192 tokens the plain kernel has no ring to fill (129 x 7,168: 8.7
+  // against 9.6 us)
+  if (tokens > 192 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && row_stride % 8 == 0 &&
+      width % 128 == 0) {
+    const uint32_t total = width / kSlab, per_xcd = div_up(total, 8);
+    hipLaunchKernelGGL(k_rope_colmean<false>, dim3(8 * per_xcd), dim3(kColmeanThreads), 0, stream,
+                       x, nullptr, nullptr, nullptr, nullptr, mean, tokens, row_stride, 0u, 0u,
+                       total, per_xcd, elem);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_colmean, dim3(div_up(width, 64)), dim3(64), 0, stream, x, mean, tokens,
                      width, row_stride, elem);
   return hipGetLastError();
@@ -967,7 +1212,7 @@ hipError_t launch_rope_colmean(const h3_prepare_cfg& cfg, uint32_t tokens, const
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const uint32_t total = cfg.heads * kSlabs, per_xcd = div_up(total, 8);
-  hipLaunchKernelGGL(k_rope_colmean, dim3(8 * per_xcd), dim3(kColmeanThreads), 0, stream, x,
+  hipLaunchKernelGGL(k_rope_colmean<true>, dim3(8 * per_xcd), dim3(kColmeanThreads), 0, stream, x,
                      weight, cos_t,
                      sin_t, r_scratch, mean, tokens, cfg.row_stride, cfg.head_offset,
                      cfg.token_capacity, total, per_xcd, cfg.elem);

@@ -233,21 +233,23 @@ int h3_stack_attend_fused(h3_stack* s, uint32_t t, h3_view fused, h3_view qnorm,
       (st = require(stage, 3, sin_t, rows * 48 * 4)) ||
       (st = require("attention", 5, out, rows * s->attention.out_stride * 2)))
     return st;
-  // Three branches (src/stack.rs:1751-1813): Q on the caller's stream, K and the V transpose on
-  // the side streams, all joined before the attention.
+  if (!s->smooth) {  // Q, K and V^T (the reference's three branches) by one launch
+    if ((st = prepare_fused(&s->prep_q, &s->prep_k, &s->transpose, t, fused, qnorm, knorm, cos_t,
+                            sin_t, s->qi, s->qs, s->ki, s->ks, s->vt, stream)))
+      return st;
+    return stack_attention(s, t, out, stream);
+  }
+  // With smoothing, three branches (src/stack.rs:1751-1813): Q on the caller's stream, K (whose
+  // column chains leave most of the chip free) and the V transpose on the side streams, all joined
+  // before the attention.
   hipStream_t caller = reinterpret_cast<hipStream_t>(stream);
   if ((st = fork_branches(s, caller))) return st;
   h3_stream k_branch = reinterpret_cast<h3_stream>(s->side[0]);
   h3_stream v_branch = reinterpret_cast<h3_stream>(s->side[1]);
   st = h3_prepare_qk_rope_i8hm(&s->prep_q, t, fused, qnorm, cos_t, sin_t, s->qi, s->qs, stream);
-  if (!st) {
-    if (s->smooth)
-      st = h3_prepare_k_rope_smooth_i8hm(&s->prep_k, t, fused, knorm, cos_t, sin_t, s->kmean,
-                                         s->ki, s->ks, k_branch);
-    else
-      st = h3_prepare_qk_rope_i8hm(&s->prep_k, t, fused, knorm, cos_t, sin_t, s->ki, s->ks,
-                                   k_branch);
-  }
+  if (!st)
+    st = h3_prepare_k_rope_smooth_i8hm(&s->prep_k, t, fused, knorm, cos_t, sin_t, s->kmean, s->ki,
+                                       s->ks, k_branch);
   // "fused V transpose" (src/stack.rs:1599-1610): workload [t]
   if (!st) st = h3_transpose_qkv_v_f16(&s->transpose, t, t, fused, s->vt, v_branch);
   const int joined = join_branches(s, caller);
@@ -316,16 +318,12 @@ int h3_stack_attend(h3_stack* s, uint32_t t, h3_view q, h3_view k, h3_view v, h3
   if (s->smooth) {  // src/stack.rs:1727-1740
     if ((st = h3_colmean_f32((uint32_t)inner, s->d.elem, t, k, s->kmean, stream))) return st;
   }
-  const h3_view kmean = s->smooth ? s->kmean : s->zmean;
-  if (s->head_major) {
-    if ((st = h3_prepare_qk_i8hm(&pq, t, q, s->zmean, s->qi, s->qs, stream))) return st;
-    if ((st = h3_prepare_qk_i8hm(&pk, t, k, kmean, s->ki, s->ks, stream))) return st;
-  } else {
-    if ((st = h3_prepare_qk_i8(&pq, t, q, s->zmean, s->qi, s->qs, stream))) return st;
-    if ((st = h3_prepare_qk_i8(&pk, t, k, kmean, s->ki, s->ks, stream))) return st;
-  }
-  // V^T over the whole capacity clears the tail (src/stack.rs:1799-1811)
-  if ((st = h3_transpose_f16(&s->transpose, s->capacity, t, v, s->vt, stream))) return st;
+  // Q and K quantized and V transposed by one launch; V^T over the whole capacity clears the tail
+  // (src/stack.rs:1799-1811)
+  if ((st = prepare_separate(&pq, &pk, &s->transpose, s->head_major, t, q, k, v,
+                             s->smooth ? s->kmean : h3_view{}, s->qi, s->qs, s->ki, s->ks, s->vt,
+                             stream)))
+    return st;
   return stack_attention(s, t, out, stream);
 }
 
