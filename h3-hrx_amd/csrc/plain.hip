@@ -14,6 +14,8 @@
 // (-ffp-contract=off; the cross-lane form below rewrites them only with exact identities).
 // Rows of up to 4096 channels take one wave each (four rows per 256-thread workgroup); wider
 // rows take one workgroup of width/64 lanes with the absmax combined through LDS.
+#include <algorithm>
+
 #include "internal.hpp"
 
 namespace h3 {
@@ -177,13 +179,10 @@ __global__ __launch_bounds__(kWide ? 512 : 256) void k_prepare_plain(
 }
 
 // 16-bit rows of up to 4,096 channels: one wave per row as k_prepare_plain<false>, but each wave
-// walks kRowsPerWave rows (row0, row0 + stride, ...) and loads the next row's inputs (8 x 16
+// walks up to kRowsPerWave rows (row0, row0 + stride, ...) and loads the next row's inputs (8 x 16
 // bytes per lane) while it transforms the current one, so a row's loads are in flight under the
 // arithmetic of the previous row.
-#ifndef H3_PLAIN_ROWS_PER_WAVE
-#define H3_PLAIN_ROWS_PER_WAVE 8
-#endif
-constexpr uint32_t kRowsPerWave = H3_PLAIN_ROWS_PER_WAVE;
+constexpr uint32_t kRowsPerWave = 8;  // at most
 
 __global__ __launch_bounds__(256) void k_prepare_plain_rows(const uint16_t* __restrict__ x,
                                                             uint32_t tokens, uint32_t width,
@@ -232,7 +231,11 @@ hipError_t launch_prepare_plain(uint32_t width, uint32_t out_stride, uint32_t el
                                 hipStream_t stream) {
   const uint32_t groups = width / kGroup;
   if (groups <= 64 && elem != H3_ELEM_F32) {
-    const uint32_t waves = (tokens + kRowsPerWave - 1) / kRowsPerWave;
+    // eight waves per CU before a wave takes more rows: with eight each, a few hundred tokens were a
+    // serial walk on a few CUs (595 tokens of 1,024 channels 25 -> 9 us, 1,500 of 4,096 29 -> 9,
+    // 5,000 of 4,096 32 -> 22)
+    const uint32_t rows = std::min(kRowsPerWave, std::max(1u, tokens / (8 * device_cus())));
+    const uint32_t waves = (tokens + rows - 1) / rows;
     hipLaunchKernelGGL(k_prepare_plain_rows, dim3((waves + 3) / 4), dim3(256), 0, stream,
                        static_cast<const uint16_t*>(x), tokens, width, out_stride, (int)elem,
                        codes, scales);

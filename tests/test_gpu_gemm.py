@@ -118,3 +118,33 @@ def test_dit_projection_shape_on_sampled_tokens(dev, m):
     assert np.array_equal(got_qk, want[:, :qk])
     assert np.array_equal(vt[:, rows].T, want[:, qk:])
     assert np.all(vt[:, m:] == 0)
+
+
+# (tokens, channels) of every way the projection is tiled (32-token workgroups, 64 x 128, 128 x 128
+# on four and on two ring stages at full and partial last tiles, 256 x 256), with step counts below,
+# at and past the rings' lengths and a 64-byte K tail
+@pytest.mark.parametrize("k", [64, 128, 192, 384, 512, 704])
+@pytest.mark.parametrize("tokens,n", [(1, 384), (32, 1152), (33, 384), (100, 8448), (200, 21504),
+                                      (520, 12288), (1100, 21504), (1500, 21504)])
+def test_every_tiling_is_bit_exact(dev, tokens, n, k):
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(tokens + n + k)
+    stride = k + 64  # bytes past K are read by no tiling
+    a = torch.randint(-128, 128, (tokens, stride), generator=g, device=dev, dtype=torch.int8)
+    w = torch.randint(-128, 128, (n, stride), generator=g, device=dev, dtype=torch.int8)
+    ws = torch.rand(n, generator=g, device=dev) + 0.5
+    scales = (torch.rand(tokens, generator=g, device=dev) + 0.5) * 1e-3
+    out = torch.full((H.compact_qkv_elements(tokens, n) + 64,), float("nan"), dtype=torch.float16,
+                     device=dev)
+    print(f"gemm tiling tokens={tokens} n={n} k={k}", flush=True)
+    H.gemm_i8_qkv_256(H.GemmCfg(k, n, stride, 4), tokens, a, w, ws, scales, out[:-64])
+    acc = a[:, :k].double() @ w[:, :k].double().t()  # exact: below 2^53
+    v = (acc.float() * ws) * scales[:, None] + 0.0   # |acc| < 2^24: exact in f32 as in the kernel
+    v = v.clamp(-65472.0, 65472.0).half()
+    cap, two = -(-tokens // 256) * 256, 2 * n // 3
+    vt = torch.zeros((n - two, cap), dtype=torch.float16, device=dev)
+    vt[:, :tokens] = v[:, two:].t()
+    want = torch.cat([v[:, :two].reshape(-1), vt.reshape(-1)])
+    assert torch.equal(out[:-64].view(torch.int16), want.view(torch.int16))
+    assert torch.isnan(out[-64:]).all(), "written past the output"
