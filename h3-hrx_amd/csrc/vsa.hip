@@ -192,23 +192,27 @@ __device__ __forceinline__ uint32_t order_key(float f) {
 // NaN patterns map below the key of -inf (0x007fffff) or above the key of +inf (0xff800000).
 __device__ __forceinline__ bool key_is_nan(uint32_t k) { return k < 0x007fffffu || k > 0xff800000u; }
 
-// h3_vsa_route: one workgroup per (q, head) row. Four 8-bit radix passes find the topk-th
-// largest candidate key (candidates: j >= prefix, not NaN); the row is then written. kPer > 0:
-// each thread keeps the keys of its candidates j = prefix + tid + kThreads*i (i < kPer) in
-// registers, so the row is read from memory once instead of once per pass.
+// h3_vsa_route: one workgroup per (q, head) row. A radix select finds T, the topk-th largest candidate
+// key (candidates: j >= prefix, not NaN); the row is then written. The digits are those of k - low over
+// the row's own range of keys, 8 bits a pass: over the keys' own bits nearly every candidate shares its
+// leading byte (sign and exponent) and the histogram's atomics collide (65 us a call at 32 heads x
+// 387 blocks and 828 at 32 x 2,112; 46 and 486 so). A pass ends the search when the threshold's bin is
+// wanted whole. kPer > 0: each thread keeps the keys of its candidates j = prefix + tid + kThreads*i
+// (i < kPer) in registers, so the row is read from memory once instead of once per pass.
 template <int kPer>
 __global__ __launch_bounds__(kThreads) void k_vsa_route(const float* __restrict__ scores,
                                                         int32_t* __restrict__ routes,
                                                         uint32_t blocks, uint32_t prefix,
                                                         uint32_t topk) {
+  constexpr int kWavesR = kThreads / 64;
   __shared__ uint32_t hist[256];
-  __shared__ uint32_t sel[3];  // chosen digit, rank left inside it, candidates (pass 0)
+  __shared__ uint32_t ends[3][kWavesR];  // each wave's lowest and highest key, and its candidates
+  __shared__ uint32_t sel[3];            // chosen digit, rank left inside it, keys inside it
   const uint32_t q = blockIdx.x, h = blockIdx.y;
   const float* row = scores + ((size_t)h * blocks + q) * blocks;
   int32_t* out = routes + ((size_t)h * blocks + q) * blocks;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const bool select = topk > 0 && q >= prefix;  // a prefix row keeps everything
-  uint32_t want = topk, bits = 0, mask = 0, candidates = 0;
   uint32_t cache[kPer > 0 ? kPer : 1];  // order keys of this thread's candidates (0: a NaN key)
   if constexpr (kPer > 0) {
 #pragma unroll
@@ -217,62 +221,94 @@ __global__ __launch_bounds__(kThreads) void k_vsa_route(const float* __restrict_
       cache[i] = j < blocks ? order_key(row[j]) : 0u;
     }
   }
-  for (int pass = 0; pass < 4 && select; ++pass) {
-    const int shift = 24 - 8 * pass;
-    hist[tid] = 0;
-    __syncthreads();
+  auto each_key = [&](auto&& use) __attribute__((always_inline)) {  // this thread's candidates
     if constexpr (kPer > 0) {
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        const uint32_t k = cache[i];
-        if (!key_is_nan(k) && (k & mask) == bits) atomicAdd(&hist[(k >> shift) & 255u], 1u);
-      }
+      for (int i = 0; i < kPer; ++i)
+        if (!key_is_nan(cache[i])) use(cache[i]);
     } else {
       for (uint32_t j = prefix + tid; j < blocks; j += kThreads) {
         const uint32_t k = order_key(row[j]);
-        if (!key_is_nan(k) && (k & mask) == bits) atomicAdd(&hist[(k >> shift) & 255u], 1u);
+        if (!key_is_nan(k)) use(k);
       }
     }
+  };
+  uint32_t low = 0, candidates = 0;  // low ends as T
+  if (select) {
+    uint32_t lo = 0xffffffffu, hi = 0u, n = 0;
+    each_key([&](uint32_t k) {
+      lo = min(lo, k);
+      hi = max(hi, k);
+      ++n;
+    });
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+      n += (uint32_t)__shfl_xor((int)n, o);
+    }
+    if (lane == 0) {
+      ends[0][tid >> 6] = lo;
+      ends[1][tid >> 6] = hi;
+      ends[2][tid >> 6] = n;
+    }
+    hist[tid] = 0;
     __syncthreads();
-    if (tid < 64) {  // lane l scans bins 255-4l, 254-4l, 253-4l, 252-4l (descending)
-      uint32_t c[4];
+    lo = ends[0][0];
+    hi = ends[1][0];
+    n = ends[2][0];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] = hist[255 - 4 * lane - i];
-      const uint32_t own = c[0] + c[1] + c[2] + c[3];
-      uint32_t incl = own;
+    for (int w = 1; w < kWavesR; ++w) {
+      lo = min(lo, ends[0][w]);
+      hi = max(hi, ends[1][w]);
+      n += ends[2][w];
+    }
+    candidates = n;
+    low = lo;
+    uint32_t want = topk, span = hi - lo;  // keys low .. low + span
+    const int bits = span ? 32 - __clz((int)span) : 0;
+    int shift = bits > 8 ? bits - 8 : 0;
+    bool more = n >= topk;  // fewer candidates than the budget: every non-NaN score stays
+    while (more) {  // uniform over the workgroup: at most four passes
+      each_key([&](uint32_t k) {
+        if (k - low <= span) atomicAdd(&hist[(k - low) >> shift], 1u);
+      });
+      __syncthreads();
+      if (tid < 64) {  // lane l scans bins 255-4l, 254-4l, 253-4l, 252-4l (descending)
+        uint32_t c[4];
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t up = __shfl_up(incl, o);
-        if ((int)lane >= o) incl += up;
-      }
-      const uint32_t excl = incl - own;
-      const uint32_t total = __shfl(incl, 63);
-      if (lane == 0 && pass == 0) sel[2] = total;
-      if (excl < want && want <= incl) {
-        uint32_t acc = excl;
+        for (int i = 0; i < 4; ++i) c[i] = hist[255 - 4 * lane - i];
+        const uint32_t own = c[0] + c[1] + c[2] + c[3];
+        uint32_t incl = own;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (acc + c[i] >= want) {
-            sel[0] = 255 - 4 * lane - i;
-            sel[1] = want - acc;
-            break;
+        for (int o = 1; o < 64; o <<= 1) {
+          const uint32_t up = __shfl_up(incl, o);
+          if ((int)lane >= o) incl += up;
+        }
+        const uint32_t excl = incl - own;
+        if (excl < want && want <= incl) {
+          uint32_t acc = excl;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (acc + c[i] >= want) {
+              sel[0] = 255 - 4 * lane - i;
+              sel[1] = want - acc;
+              sel[2] = c[i];
+              break;
+            }
+            acc += c[i];
           }
-          acc += c[i];
         }
       }
+      __syncthreads();
+      low += sel[0] << shift;
+      want = sel[1];
+      more = shift > 0 && sel[2] != want;  // the whole bin is wanted: its lowest key will do
+      span = (1u << shift) - 1;
+      shift = shift > 8 ? shift - 8 : 0;
+      hist[tid] = 0;
+      __syncthreads();
     }
-    __syncthreads();
-    if (pass == 0) {
-      candidates = sel[2];
-      if (candidates < want) {  // fewer candidates than the budget: every non-NaN score stays
-        __syncthreads();
-        break;
-      }
-    }
-    bits |= sel[0] << shift;
-    mask |= 255u << shift;
-    want = sel[1];
-    __syncthreads();
   }
   const bool all = select && candidates < topk;
   // routes[q][j]: 1 when forced (a prefix row or column, |q - j| <= 1); else 0 without a budget,
@@ -280,7 +316,7 @@ __global__ __launch_bounds__(kThreads) void k_vsa_route(const float* __restrict_
   auto keep_of = [&](uint32_t j, uint32_t k) -> int32_t {
     if (q < prefix || j < prefix || (j <= q + 1 && q <= j + 1)) return 1;
     if (topk == 0) return 0;
-    return all || key_is_nan(k) || k >= bits ? 1 : 0;
+    return all || key_is_nan(k) || k >= low ? 1 : 0;
   };
   if constexpr (kPer > 0) {
     for (uint32_t j = tid; j < prefix && j < blocks; j += kThreads) out[j] = 1;
@@ -296,62 +332,82 @@ __global__ __launch_bounds__(kThreads) void k_vsa_route(const float* __restrict_
 
 // h3_vsa_coarse: coarse[q][128h+c] = sum_j w_qj vm[j][128h+c] / sum_j w_qj with
 // w_qj = exp(scores[h][q][j]*scale - max_j(scores[h][q][j]*scale)), the max starting at -1e9.
-// A workgroup takes 32 query blocks of one head; thread (c, g) owns channel c of 16 of them.
-constexpr int kCoarseRows = 32;
-constexpr int kCoarseCols = 64;  // key blocks per LDS slice
+// A workgroup takes 16 query blocks of one head; thread (c, g) owns channel c of 8 of them and takes
+// the key blocks four at a time (a fma chain over them in order), with sixteen values of its column in
+// flight and one 16-byte weight read per row and four blocks. One key block at a time, with a 4-byte
+// weight read per product and one column load in flight, took 188 us at 32 heads x 387 blocks; 60 so.
+constexpr int kCoarseRows = 16;
+constexpr int kCoarseCols = 64;            // key blocks per LDS slice
+constexpr int kCoarsePad = kCoarseCols + 4;
+constexpr int kRowThreads = kThreads / kCoarseRows;  // threads per row for the max and the weights
 __global__ __launch_bounds__(kThreads) void k_vsa_coarse(const float* __restrict__ scores,
                                                          const float* __restrict__ vm,
                                                          float* __restrict__ coarse,
                                                          uint32_t blocks, uint32_t width) {
-  __shared__ float w[kCoarseRows][kCoarseCols + 1];
-  __shared__ float row_max[kCoarseRows];
+  __shared__ __attribute__((aligned(16))) float w[kCoarseRows][kCoarsePad];
   __shared__ float row_sum[kCoarseRows];
   const float scale = 0.08838834764831845f;
   const uint32_t h = blockIdx.y, q0 = blockIdx.x * kCoarseRows;
   const uint32_t tid = threadIdx.x;
-  // max: 8 threads per row
-  const uint32_t r8 = tid >> 3, p8 = tid & 7;
-  const float* srow = scores + ((size_t)h * blocks + q0 + r8) * blocks;
-  const bool row_live = q0 + r8 < blocks;
+  const uint32_t rr = tid / kRowThreads, pr = tid % kRowThreads;
+  const float* srow = scores + ((size_t)h * blocks + q0 + rr) * blocks;
+  const bool row_live = q0 + rr < blocks;
   float m = -1.0e9f;
   if (row_live)
-    for (uint32_t j = p8; j < blocks; j += 8) m = fmaxf(srow[j] * scale, m);
+    for (uint32_t j = pr; j < blocks; j += kRowThreads) m = fmaxf(srow[j] * scale, m);
 #pragma unroll
-  for (int o = 1; o < 8; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+  for (int o = 1; o < kRowThreads; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
   float part = 0.0f;  // this thread's share of the row sum
   const uint32_t c = tid & 127, g = tid >> 7;
-  float acc[16] = {};
+  constexpr int kOwn = kCoarseRows / 2;
+  float acc[kOwn] = {};
   const float* vcol = vm + (size_t)h * 128 + c;
-  for (uint32_t j0 = 0; j0 < blocks; j0 += kCoarseCols) {
-    // weights of the slice: 8 threads per row, 8 key blocks each
+  // sixteen values of the column, requested sixteen key blocks ahead (0 past the last block, where the
+  // weights are 0 too)
+  constexpr int kAhead = 16;
+  float cur[kAhead], nxt[kAhead];
+  auto request = [&](float (&v)[kAhead], uint32_t j) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kCoarseCols / 8; ++i) {
-      const uint32_t jj = p8 * (kCoarseCols / 8) + i, j = j0 + jj;
+    for (int x = 0; x < kAhead; ++x) v[x] = j + x < blocks ? vcol[(size_t)(j + x) * width] : 0.0f;
+  };
+  request(cur, 0);
+  for (uint32_t j0 = 0; j0 < blocks; j0 += kCoarseCols) {
+#pragma unroll
+    for (int i = 0; i < kCoarseCols / kRowThreads; ++i) {
+      const uint32_t jj = pr + kRowThreads * i, j = j0 + jj;
       float wv = 0.0f;
       if (row_live && j < blocks) wv = __expf(srow[j] * scale - m);
       part += wv;
-      w[r8][jj] = wv;
+      w[rr][jj] = wv;
     }
     __syncthreads();
-    const uint32_t jn = blocks - j0 < (uint32_t)kCoarseCols ? blocks - j0 : kCoarseCols;
-    for (uint32_t jj = 0; jj < jn; ++jj) {
-      const float v = vcol[(size_t)(j0 + jj) * width];
+#pragma unroll 1
+    for (int jj = 0; jj < kCoarseCols; jj += kAhead) {
+      request(nxt, j0 + jj + kAhead);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(w[16 * g + i][jj], v, acc[i]);
+      for (int x = 0; x < kAhead; x += 4) {
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+          const float4 w4 = *reinterpret_cast<const float4*>(&w[kOwn * g + i][jj + x]);
+          acc[i] = __builtin_fmaf(w4.x, cur[x], acc[i]);
+          acc[i] = __builtin_fmaf(w4.y, cur[x + 1], acc[i]);
+          acc[i] = __builtin_fmaf(w4.z, cur[x + 2], acc[i]);
+          acc[i] = __builtin_fmaf(w4.w, cur[x + 3], acc[i]);
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < kAhead; ++x) cur[x] = nxt[x];
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int o = 1; o < 8; o <<= 1) part += __shfl_xor(part, o);
-  if (p8 == 0) {
-    row_max[r8] = m;
-    row_sum[r8] = part;
-  }
+  for (int o = 1; o < kRowThreads; o <<= 1) part += __shfl_xor(part, o);
+  if (pr == 0) row_sum[rr] = part;
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t q = q0 + 16 * g + i;
-    if (q < blocks) coarse[(size_t)q * width + (size_t)h * 128 + c] = acc[i] / row_sum[16 * g + i];
+  for (int i = 0; i < kOwn; ++i) {
+    const uint32_t q = q0 + kOwn * g + i;
+    if (q < blocks) coarse[(size_t)q * width + (size_t)h * 128 + c] = acc[i] / row_sum[kOwn * g + i];
   }
 }
 
@@ -385,15 +441,36 @@ __global__ __launch_bounds__(kThreads) void k_vsa_gated_scatter(
   }
 }
 
-// h3_vsa_kmean: mean[c] = (sum_t x[t][c]) / f32(tokens), a running f32 sum over the rows.
-__global__ __launch_bounds__(kThreads) void k_vsa_kmean(const float* __restrict__ x,
-                                                        float* __restrict__ mean,
-                                                        uint32_t tokens, uint32_t width) {
-  const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+// h3_vsa_kmean: mean[c] = (sum_t x[t][c]) / f32(tokens), a running f32 sum over the rows. One wave per
+// 64 columns, 32 loads in flight ahead of the dependent adds (eight, in workgroups of 256 columns:
+// 129 us at 2,112 x 4,096, 54 so; 20 and 9 at 259 x 2,048).
+constexpr int kMeanThreads = 64;
+constexpr uint32_t kMeanAhead = 32;
+__global__ __launch_bounds__(kMeanThreads) void k_vsa_kmean(const float* __restrict__ x,
+                                                            float* __restrict__ mean,
+                                                            uint32_t tokens, uint32_t width) {
+  const uint32_t c = blockIdx.x * kMeanThreads + threadIdx.x;
   if (c >= width) return;
+  const float* p = x + c;
   float acc = 0.0f;
-#pragma unroll 8
-  for (uint32_t t = 0; t < tokens; ++t) acc = acc + x[(size_t)t * width + c];
+  float cur[kMeanAhead], nxt[kMeanAhead];
+  auto load = [&](float (&v)[kMeanAhead], uint32_t t) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < kMeanAhead; ++i) v[i] = p[(size_t)(t + i) * width];
+  };
+  uint32_t t = 0;
+  if (tokens >= kMeanAhead) load(cur, 0);
+  for (; t + kMeanAhead <= tokens; t += kMeanAhead) {
+    const bool more = t + 2 * kMeanAhead <= tokens;  // uniform
+    if (more) load(nxt, t + kMeanAhead);
+#pragma unroll
+    for (uint32_t i = 0; i < kMeanAhead; ++i) acc = acc + cur[i];
+    if (more) {
+#pragma unroll
+      for (uint32_t i = 0; i < kMeanAhead; ++i) cur[i] = nxt[i];
+    }
+  }
+  for (; t < tokens; ++t) acc = acc + p[(size_t)t * width];
   mean[c] = acc / (float)tokens;
 }
 
@@ -476,8 +553,8 @@ hipError_t launch_vsa_gated_scatter(uint32_t tokens, uint32_t padded, uint32_t w
 
 hipError_t launch_vsa_kmean(uint32_t tokens, uint32_t width, const float* x, float* mean,
                             hipStream_t stream) {
-  hipLaunchKernelGGL(k_vsa_kmean, dim3((width + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                     stream, x, mean, tokens, width);
+  hipLaunchKernelGGL(k_vsa_kmean, dim3((width + kMeanThreads - 1) / kMeanThreads),
+                     dim3(kMeanThreads), 0, stream, x, mean, tokens, width);
   return hipGetLastError();
 }
 

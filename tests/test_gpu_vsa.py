@@ -544,3 +544,31 @@ def test_runtime_with_prefix_segments_layers_and_gate(dev):
             diff = np.abs(got.view(np.float16).astype(np.float32) - want.view(np.float16).astype(np.float32))
             assert diff.max() < 1e-2, diff.max()
     vsa.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 15, 17, 63, 64, 65, 130])
+def test_coarse_and_kmean_at_the_edges_of_their_tiles(dev, blocks):
+    """Coarse takes 16 query blocks per workgroup and the key blocks 64 per slice, 16 ahead; the K mean
+    32 rows ahead of its adds. The oracle's f64 coarse at 1e-5 of the values' size (f32 sums of up to 130
+    terms and the hardware exp), the K mean bit for bit."""
+    import torch
+
+    heads = 3
+    width = heads * 128
+    rng = np.random.default_rng(blocks)
+    scores = (rng.standard_normal((heads, blocks, blocks)) * 20).astype(np.float32)
+    vm = rng.standard_normal((blocks, width)).astype(np.float32)
+    cfg = H.VsaCfg(64 * blocks, 64 * blocks, width, blocks, heads, 0, 1)
+    got = torch.full((blocks, width), float("nan"), dtype=torch.float32, device=dev)
+    print(f"coarse and kmean blocks={blocks}", flush=True)
+    H.vsa_coarse(cfg, to_dev(scores, dev), to_dev(vm, dev), got)
+    x = scores.astype(np.float64) * 0.08838834764831845
+    w = np.exp(x - x.max(2, keepdims=True))
+    w /= w.sum(2, keepdims=True)
+    want = np.concatenate([w[h] @ vm[:, 128 * h:128 * h + 128].astype(np.float64)
+                           for h in range(heads)], 1)
+    assert np.abs(got.cpu().numpy() - want).max() <= 1e-5 * max(1.0, np.abs(vm).max())
+    mean = torch.empty(width, dtype=torch.float32, device=dev)
+    H.vsa_kmean(width, blocks, to_dev(vm, dev), mean)
+    total = np.add.accumulate(vm, axis=0, dtype=np.float32)[-1]
+    assert np.array_equal(mean.cpu().numpy(), total / np.float32(blocks))
