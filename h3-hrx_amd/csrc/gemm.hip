@@ -220,15 +220,17 @@ __device__ __forceinline__ void tile(const Args& a, uint32_t m0, uint32_t n0, ch
     read_operands(op, nxt, 0, arow, wrow, half, sw);  // after the last step: unused
     const Loads l = loads_of(i + kRing);
     __builtin_amdgcn_sched_barrier(0);
-    // The loads of step i + kRing, one behind each MFMA where there is one for each: a wave takes about
-    // 65 cycles to issue one, which in a burst ahead of the MFMAs left the matrix cores idle (256 x
-    // 256 tiles: 1,543 -> 1,521 us at 31,104 tokens, 6,447 -> 6,343 at 129,024, with the barrier
-    // moved). Smaller tiles have fewer MFMAs than loads and run 2 % better with the burst.
+    // The loads of step i + kRing, two behind each of the first MFMAs: a wave takes about 65 cycles to
+    // issue one, which in a burst ahead of the MFMAs left the matrix cores idle (256 x 256 tiles: 1,543
+    // -> 1,521 us at 31,104 tokens, 6,447 -> 6,343 at 129,024, with the barrier moved; one behind each
+    // of the eight leaves the last ones less time to land, 2 % slower where the operands come from
+    // HBM). Smaller tiles have fewer MFMAs than loads and run 2 % better with the burst.
     if constexpr (kMB * kNB >= T::kLoads) {
 #pragma unroll
       for (int x = 0; x < kMB * kNB; ++x) {
         mma_one<kTrans>(op, 3, x / kNB, x % kNB, acc);
-        if (x < T::kLoads) load(l, cur, x);
+#pragma unroll
+        for (int t = 2 * x; t < 2 * x + 2 && t < T::kLoads; ++t) load(l, cur, t);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
@@ -461,13 +463,16 @@ hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_str
   if (m <= 32) return launch_few(g, stream);
   // The tile that prices lowest, in us per 128 bytes of K (n: tiles with tokens in them, per CU).
   // Measured:
-  //   256 x 256          1.5 + n in the first round of one tile per CU, 2.15 per round after it
-  //   128 x 128, ring 2  two per CU: 1.05 up to 1.5 each, 1.9 up to two, 0.6 + 0.54 n
+  //   256 x 256          1.5 + n in the first round of one tile per CU, 2.15 per round up to three,
+  //                      2.35 n
+  //   128 x 128, ring 2  two per CU: 1.05 up to 1.5 each, 1.9 up to two, 0.6 + 0.54 n up to eight,
+  //                      0.66 n
   //   128 x 128, ring 4  one per CU, its loads four steps ahead: 0.66 up to one each, 0.55 + 0.55 n
   //                      where it is not past three and a half rounds
   //   64 x 128, ring 4   where even those leave three CUs of four idle
   // At K = 4,096, N = 12,288 (us: 256 x 256 / 128 x 128 ring 2 / ring 4): 64 tokens 51 / 27 / 19, 300
-  // 63 / 33 / 39, 513 64 / 62 / 59, 1,024 73 / 67 / 66, 2,048 137 / 117 / 125, 5,000 253 / 284 / 303;
+  // 63 / 33 / 39, 513 64 / 62 / 59, 1,024 73 / 67 / 66, 2,048 137 / 117 / 125, 5,000 253 / 284 / 303, 12,000 at
+  // N = 7,680, K = 3,072 314 / 350 (ring 2);
   // 200 tokens at N = 1,536, K = 2,816: 45 / 17 / 16, 12 on 64 x 128.
   const float cus = device_cus();
   auto tiles = [&](uint32_t bm, uint32_t bn) {
@@ -476,8 +481,8 @@ hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_str
   };
   const float n0 = tiles(256, 256), n1 = tiles(128, 128);
   if (tiles(64, 128) <= 0.25f) return launch_tiles<1, 1, 4>(g, stream);
-  const float t0 = n0 <= 1.0f ? 1.5f + n0 : 2.15f * std::ceil(n0);
-  const float t2 = n1 <= 1.5f ? 1.05f : n1 <= 2.0f ? 1.9f : 0.6f + 0.54f * n1;
+  const float t0 = n0 <= 1.0f ? 1.5f + n0 : n0 <= 3.0f ? 2.15f * std::ceil(n0) : 2.35f * n0;
+  const float t2 = n1 <= 1.5f ? 1.05f : n1 <= 2.0f ? 1.9f : n1 <= 8.0f ? 0.6f + 0.54f * n1 : 0.66f * n1;
   const float t4 = n1 <= 1.0f ? 0.66f : n1 <= 1.5f ? 1.25f : n1 <= 3.5f ? 0.55f + 0.55f * n1 : 1e9f;
   if (t0 <= t2 && t0 <= t4) return launch_tiles<4, 2, 2>(g, stream);
   return t2 <= t4 ? launch_tiles<2, 1, 2>(g, stream) : launch_tiles<2, 1, 4>(g, stream);

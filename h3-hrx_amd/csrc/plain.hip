@@ -231,10 +231,12 @@ hipError_t launch_prepare_plain(uint32_t width, uint32_t out_stride, uint32_t el
                                 hipStream_t stream) {
   const uint32_t groups = width / kGroup;
   if (groups <= 64 && elem != H3_ELEM_F32) {
-    // eight waves per CU before a wave takes more rows: with eight each, a few hundred tokens were a
-    // serial walk on a few CUs (595 tokens of 1,024 channels 25 -> 9 us, 1,500 of 4,096 29 -> 9,
-    // 5,000 of 4,096 32 -> 22)
-    const uint32_t rows = std::min(kRowsPerWave, std::max(1u, tokens / (8 * device_cus())));
+    // Rows per wave so that the waves come to eight per CU, evenly: with eight rows each, a few
+    // hundred tokens were a serial walk on a few CUs (595 tokens of 1,024 channels 25 -> 9 us, 1,500
+    // of 4,096 29 -> 9, 5,000 32 -> 22), and a few waves more than eight per CU leave some with half as
+    // much again (16,000 of 4,096: seven rows a wave 54 us, eight 46).
+    const uint32_t even = 8 * device_cus();
+    const uint32_t rows = std::min(kRowsPerWave, (tokens + even - 1) / even);
     const uint32_t waves = (tokens + rows - 1) / rows;
     hipLaunchKernelGGL(k_prepare_plain_rows, dim3((waves + 3) / 4), dim3(256), 0, stream,
                        static_cast<const uint16_t*>(x), tokens, width, out_stride, (int)elem,
