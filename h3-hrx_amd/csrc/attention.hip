@@ -1745,14 +1745,24 @@ size_t vsa_part_bytes(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t*
 // generation of resident workgroups: its workgroups start together and walk their ascending key
 // lists at about the same pace, so more of the tiles they share are still in L2 (measured at 129k
 // tokens with token-major scales: 45.9 ms against 56.5 ms for one launch of all the work).
+// A call of short lists over few key cubes is one launch all the same: an XCD's L2 then holds most
+// of what its heads share at any pace, and each generation's end leaves CUs idle for the length of
+// a walk. Whole runtime, one launch against generations, INT8 and 16-bit Q/K: 17,550 tokens x 32
+// heads keeping 44 cubes 1,441 against 1,551 us and 1,486 against 1,614; 9,145 x 24 keeping 50 723
+// against 781 and 723 against 801; 30,000 x 32 (527 key cubes) keeping 35 2,261 against 2,352 and
+// 2,551 against 2,582. Beyond either limit generations win: 61,440 x 24 (960 cubes) keeping 31
+// 3,113 against 3,169 and 3,261 against 3,463; 17,550 x 8 keeping 78 624 against 631 and 640
+// against 677; 129,024 x 32 34.8 against 45.8 ms and 47.5 against 60.8.
+static constexpr uint32_t kOneLaunchKept = 64, kOneLaunchBlocks = 640;
+
 template <bool kHmScales, bool kF16>
 static hipError_t launch_vsa_cubes(Args a, uint32_t heads, const VsaPrefix& prefix,
                                    hipStream_t stream) {
   const uint32_t all = a.q_blocks, gen = vsa_generation();
-  auto generations = [&](uint32_t items, auto kernel) {
-    for (uint32_t base = 0; base < items; base += gen) {
+  auto launches = [&](uint32_t items, uint32_t size, auto kernel) {
+    for (uint32_t base = 0; base < items; base += size) {
       a.base = base;
-      a.total = std::min(gen, items - base);
+      a.total = std::min(size, items - base);
       a.per_xcd = (a.total + 7) / 8;
       hipLaunchKernelGGL(kernel, dim3(a.per_xcd * 8), dim3(kVsaThreads), 0, stream, a);
     }
@@ -1764,18 +1774,20 @@ static hipError_t launch_vsa_cubes(Args a, uint32_t heads, const VsaPrefix& pref
     a.part = prefix.part;
     if (prefix.splits > 1) {
       if constexpr (kHmScales || kF16) {  // the runtime's two forms
-        generations(first * heads * prefix.splits, k_attention_vsa<kHmScales, kF16, true>);
+        launches(first * heads * prefix.splits, gen, k_attention_vsa<kHmScales, kF16, true>);
         hipLaunchKernelGGL(k_vsa_combine, dim3(first * heads), dim3(256), 0, stream, prefix.part,
                            a.out, first, prefix.splits, std::min(a.token_count, a.tokens),
                            a.out_stride, a.kv_head_limit, a.head_limit);
       }
     } else {
-      generations(first * heads, k_attention_vsa<kHmScales, kF16>);
+      launches(first * heads, gen, k_attention_vsa<kHmScales, kF16>);
     }
   }
   a.cube0 = first;
   a.q_blocks = all - first;
-  if (a.q_blocks > 0) generations(a.q_blocks * heads, k_attention_vsa<kHmScales, kF16>);
+  const uint32_t items = a.q_blocks * heads;
+  const bool one = prefix.kept > 0 && prefix.kept <= kOneLaunchKept && all <= kOneLaunchBlocks;
+  if (items > 0) launches(items, one ? items : gen, k_attention_vsa<kHmScales, kF16>);
   return hipGetLastError();
 }
 

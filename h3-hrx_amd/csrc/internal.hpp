@@ -179,8 +179,9 @@ hipError_t launch_attention_cross(const h3_cross_cfg& cfg, const int32_t* qi, co
 // The query cubes [0, cubes) of every head whose routes keep (nearly) every key cube, the VSA
 // runtime's prefix: their own launches, each cube split into `splits` ranges of the key cubes when
 // `splits` > 1, with the ranges' partial results in `part` (vsa_part_bytes). Empty: no such cubes.
+// `kept`: about how many key cubes each other query cube keeps (0: unknown).
 struct VsaPrefix {
-  uint32_t cubes = 0, splits = 1;
+  uint32_t cubes = 0, splits = 1, kept = 0;
   float* part = nullptr;
 };
 // The number of ranges for `cubes` prefix cubes of `heads` heads over `blocks` key cubes, and the

@@ -255,6 +255,7 @@ int h3_vsa_build_bits(const int32_t* src, const int32_t* inverse, const int32_t*
     }
   }
   r->prefix.cubes = prefix_blocks;
+  r->prefix.kept = prefix_blocks + r->cfg.topk + 2;  // the prefix, its own choice, an edge or two
   const size_t part_bytes = vsa_part_bytes(heads, prefix_blocks, blocks, &r->prefix.splits);
   if (part_bytes) {
     if ((st = allocate(&r->part, part_bytes))) {

@@ -13,12 +13,13 @@ pytestmark = pytest.mark.gpu
 
 
 # prefix rows of one partial cube, of three cubes with a partial one (splits), of more cubes than one
-# generation of workgroups takes (no split), a plan of few key cubes (fewer than eight to a range), and
-# a plan that is nearly all prefix
+# generation of workgroups takes (no split), a plan of few key cubes (fewer than eight to a range), a
+# plan that is nearly all prefix, and one whose video cubes, more than three generations of them, are
+# one launch of the runtime
 @pytest.mark.parametrize("bits", [8, 16])
 @pytest.mark.parametrize("segments,grid,heads", [
     ([(0, 5)], (8, 12, 13), 2), ([(0, 77), (77, 70)], (9, 16, 17), 3), ([(0, 2112)], (4, 16, 16), 32),
-    ([(0, 64)], (4, 8, 4), 2), ([(0, 700)], (4, 5, 4), 2)])
+    ([(0, 64)], (4, 8, 4), 2), ([(0, 700)], (4, 5, 4), 2), ([(0, 30)], (9, 25, 26), 24)])
 def test_runtime_prefix_cubes_match_the_whole_walk(dev, bits, segments, grid, heads):
     import torch
 
