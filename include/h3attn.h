@@ -595,11 +595,11 @@ uint32_t h3_stack_capacity(const h3_stack *stack);
 
 /* Stack::prepare_fused_operands (src/stack.rs:1541-1616) followed by attention: reads the fused
  * QKV projection [t][3*heads*128], per-head norm weights, cos/sin [t][48]; writes the attention
- * output [t][heads*128] f16. The Q quantizer, the K quantizer (smoothed or not) and the V
- * transpose are three independent branches, as the reference records them
- * (src/stack.rs:1751-1813): forked from `stream` onto the stack's side streams with an event and
- * joined back before the attention, so the call stays ordered on `stream` and capturable. Calls
- * on one stack must not overlap (they share its side streams and operand buffers). */
+ * output [t][heads*128] f16. The Q quantizer, the K quantizer and the V transpose, three independent
+ * branches in the reference (src/stack.rs:1751-1813), are one launch on `stream`; with smoothing, Q
+ * runs there and the smoothed K and V are forked onto the stack's side streams with an event and
+ * joined back before the attention. Either way the call stays ordered on `stream` and capturable.
+ * Calls on one stack must not overlap (they share its side streams and operand buffers). */
 int h3_stack_attend_fused(h3_stack *stack, uint32_t t, h3_view fused, h3_view qnorm,
                           h3_view knorm, h3_view cos_t, h3_view sin_t, h3_view out,
                           h3_stream stream);
