@@ -139,7 +139,7 @@ __device__ __forceinline__ void tile(const Args& a, uint32_t m0, uint32_t n0, ch
   // DMA map: load t of wave w fills stage bytes [(kLoads w + t) * 1024, + 1024), eight rows of A or
   // of W; lane l writes row r = (kLoads w + t) * 8 + l/8, position l%8, which holds logical chunk
   // (l%8) ^ ((r/2)%8).
-  const uint32_t a_left = a.m > m0 ? min(a.m - m0, (uint32_t)T::kBM) : 0u;
+  const uint32_t a_left = min(a.m - m0, (uint32_t)T::kBM);
   const uint32_t w_left = a.n > n0 ? min(a.n - n0, (uint32_t)T::kBN) : 0u;
   const int8_t* a_base = a.a + (size_t)m0 * a.k_stride;
   const int8_t* w_base = a.w + (size_t)n0 * a.k_stride;
@@ -164,7 +164,7 @@ __device__ __forceinline__ void tile(const Args& a, uint32_t m0, uint32_t n0, ch
   };
   const int8_t* own_base = is_a(0) ? a_base : w_base;
   const uint32_t own_bytes = is_a(0) ? a_bytes : w_bytes;
-  const uint32_t steps = a.m > m0 ? (a.k + kBK - 1) / kBK : 0u;  // past the tokens: zeros only
+  const uint32_t steps = (a.k + kBK - 1) / kBK;
   const bool tail = a.k % kBK != 0;
   auto loads_of = [&](uint32_t i) {  // step i; past the last step the descriptors are empty
     const uint32_t k0 = i * kBK;
@@ -320,6 +320,17 @@ __device__ __forceinline__ void tile(const Args& a, uint32_t m0, uint32_t n0, ch
         }
       }
     }
+    // The last tile of tokens also writes the zeros up to the capacity. Tiles of their own for them
+    // took slots from the others: 513 tokens x 12,288 are 480 tiles of 128 x 128, which fit two to a
+    // CU, and 96 more did not (K 4,096: 62.7 us with them, 40.5 so).
+    if (m0 + T::kBM >= a.m) {
+      const uint32_t first = m0 + T::kBM, per = (a.cap - first) / 4;
+      for (uint32_t i = threadIdx.x; i < T::kBN * per; i += kThreads) {
+        const uint32_t n = n0 + i / per;
+        if (n < a.n)
+          *reinterpret_cast<v4h*>(vt + (size_t)(n - a.qk_width) * a.cap + first + 4 * (i % per)) = v4h{};
+      }
+    }
   }
 }
 
@@ -342,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_i8_qkv(Args a) {
   const uint32_t n_tile = r / m_in;
   const uint32_t m0 = m_tile * T::kBM;
   if (n_tile < a.tiles_n_qk) {
-    if (m0 < a.m) tile<true, kMB, kNB, kRing>(a, m0, n_tile * T::kBN, s0, s1, s2, s3);
+    tile<true, kMB, kNB, kRing>(a, m0, n_tile * T::kBN, s0, s1, s2, s3);
   } else {
     tile<false, kMB, kNB, kRing>(a, m0, a.qk_width + (n_tile - a.tiles_n_qk) * T::kBN, s0, s1, s2,
                                  s3);
@@ -352,7 +363,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_i8_qkv(Args a) {
 template <int kMB, int kNB, int kRing>
 hipError_t launch_tiles(Args g, hipStream_t stream) {
   using T = Tile<kMB, kNB>;
-  g.tiles_m = g.cap / T::kBM;
+  g.tiles_m = (g.m + T::kBM - 1) / T::kBM;
   g.tiles_n_qk = (g.qk_width + T::kBN - 1) / T::kBN;
   g.tiles_n = g.tiles_n_qk + (g.n - g.qk_width + T::kBN - 1) / T::kBN;
   g.total = g.tiles_m * g.tiles_n;
@@ -461,29 +472,35 @@ hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_str
   g.qk_width = n / 3 * 2;
   g.cap = (m + kCapRows - 1) / kCapRows * kCapRows;
   if (m <= 32) return launch_few(g, stream);
-  // The tile that prices lowest, in us per 128 bytes of K (n: tiles with tokens in them, per CU).
-  // Measured:
-  //   256 x 256          1.5 + n in the first round of one tile per CU, 2.15 per round up to three,
-  //                      2.35 n
-  //   128 x 128, ring 2  two per CU: 1.05 up to 1.5 each, 1.9 up to two, 0.6 + 0.54 n up to eight,
-  //                      0.66 n
-  //   128 x 128, ring 4  one per CU, its loads four steps ahead: 0.66 up to one each, 0.55 + 0.55 n
-  //                      where it is not past three and a half rounds
-  //   64 x 128, ring 4   where even those leave three CUs of four idle
-  // At K = 4,096, N = 12,288 (us: 256 x 256 / 128 x 128 ring 2 / ring 4): 64 tokens 51 / 27 / 19, 300
-  // 63 / 33 / 39, 513 64 / 62 / 59, 1,024 73 / 67 / 66, 2,048 137 / 117 / 125, 5,000 253 / 284 / 303, 12,000 at
-  // N = 7,680, K = 3,072 314 / 350 (ring 2);
-  // 200 tokens at N = 1,536, K = 2,816: 45 / 17 / 16, 12 on 64 x 128.
-  const float cus = device_cus();
+  // The tile that prices lowest in us, s steps of 128 bytes of K: fixed costs, what a tile costs besides its
+  // steps (its fill and its epilogue, which nothing overlaps at one 256 x 256 tile per CU), and its steps.
+  // n0, n1: 256 x 256 and 128 x 128 tiles per CU. 256 x 256 run one to a CU, in rounds; 128 x 128 on a ring
+  // of two stages two to a CU; on a ring of four one, its loads four steps ahead. 64 x 128 where the others
+  // leave three CUs of four idle. Fitted to 64 to 8,192 tokens at (N, K) = (12,288, 4,096), (21,504, 7,168),
+  // (6,144, 2,048), (3,072, 5,120), (7,680, 3,072), (21,504, 1,024) and (15,360, 6,400), W in the caches and
+  // not: the choice costs 0.4 % over the best tile in the mean and 12 % at the most (prices per step of K
+  // alone: 2.9 and 47 %). Measured (us: 256 x 256 / 128 x 128 ring 2 / ring 4), at K = 4,096, N = 12,288:
+  // 129 tokens 57 / 29 / 22, 513 64 / 41 / 44, 1,025 76 / 73 / 77, 5,000 246 / 279 / 298; 2,049 at K =
+  // 1,024, N = 21,504 113 / 87 / 108; 641 at K = 7,168, N = 21,504 110 / 120 / 124.
+  const float cus = device_cus(), s = k / 128.0f;
   auto tiles = [&](uint32_t bm, uint32_t bn) {
     const uint32_t qk = (g.qk_width + bn - 1) / bn, v = (n - g.qk_width + bn - 1) / bn;
     return (m + bm - 1) / bm * (qk + v) / cus;
   };
-  const float n0 = tiles(256, 256), n1 = tiles(128, 128);
   if (tiles(64, 128) <= 0.25f) return launch_tiles<1, 1, 4>(g, stream);
-  const float t0 = n0 <= 1.0f ? 1.5f + n0 : n0 <= 3.0f ? 2.15f * std::ceil(n0) : 2.35f * n0;
-  const float t2 = n1 <= 1.5f ? 1.05f : n1 <= 2.0f ? 1.9f : n1 <= 8.0f ? 0.6f + 0.54f * n1 : 0.66f * n1;
-  const float t4 = n1 <= 1.0f ? 0.66f : n1 <= 1.5f ? 1.25f : n1 <= 3.5f ? 0.55f + 0.55f * n1 : 1e9f;
+  const float n0 = tiles(256, 256), n1 = tiles(128, 128);
+  const float rounds = n0 <= 3.0f ? 0.84f * std::ceil(n0) + 0.16f * n0 : n0 + 0.2f;
+  const float t0 = n0 <= 1.0f ? 28.75f + s * (0.89f + 0.61f * n0)
+                              : 8.91f + rounds * (19.84f + 1.43f * s);
+  const float t2 = 7.01f + 3.43f * n1 +
+                   s * (n1 <= 2.0f   ? 0.64f + 0.29f * std::max(n1 - 1.0f, 0.0f)
+                        : n1 <= 4.0f ? 1.48f + 0.18f * (n1 - 2.0f)
+                                     : 0.21f + 0.475f * n1);
+  const float t4 = 7.6f + 4.95f * n1 +
+                   s * (n1 <= 1.0f   ? 0.35f
+                        : n1 <= 2.0f ? 0.85f
+                        : n1 <= 4.0f ? 1.17f + 0.36f * (n1 - 2.0f)
+                                     : 0.1f + 0.475f * n1);
   if (t0 <= t2 && t0 <= t4) return launch_tiles<4, 2, 2>(g, stream);
   return t2 <= t4 ? launch_tiles<2, 1, 2>(g, stream) : launch_tiles<2, 1, 4>(g, stream);
 }

@@ -148,3 +148,11 @@ def test_every_tiling_is_bit_exact(dev, tokens, n, k):
     want = torch.cat([v[:, :two].reshape(-1), vt.reshape(-1)])
     assert torch.equal(out[:-64].view(torch.int16), want.view(torch.int16))
     assert torch.isnan(out[-64:]).all(), "written past the output"
+
+
+# long K, where the prices per step decide: 256 x 256 in one round and in two, 128 x 128 on four stages with
+# the capacity's last columns past the tokens' tiles and inside them, 128 x 128 on two stages
+@pytest.mark.parametrize("tokens,n,k", [(520, 21504, 6208), (1100, 21504, 7232), (257, 21504, 7232),
+                                        (900, 3072, 5184), (300, 12288, 4160)])
+def test_tilings_of_a_long_k_are_bit_exact(dev, tokens, n, k):
+    test_every_tiling_is_bit_exact(dev, tokens, n, k)
