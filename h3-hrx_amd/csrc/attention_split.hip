@@ -5,7 +5,7 @@
 //
 // k_attention_hm gives 256 queries of one head to a workgroup, which walks every key: a call of B
 // blocks takes ceil(B / CUs) rounds of a whole walk, however few blocks the last round holds. Here
-// a workgroup's eight waves are QW tiles of 32 queries times KS = 8 / QW groups of keys: group g
+// a workgroup's eight waves are QW (one or two) tiles of 32 queries times KS = 8 / QW groups of keys: group g
 // walks the 64-key stages g, g + KS, ..., each wave with an online softmax of its own, and the KS
 // partial results of a tile are combined through LDS at the end. A block's work is then spread
 // over 8 / QW workgroups, each of which takes 1 / KS of the walk, without device memory for the
@@ -381,8 +381,8 @@ SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t cu
   float best_time = std::min(0.98f * whole, whole - 1.0f);
   const uint32_t mains[2] = {full_blocks / cus * cus, full_blocks};
   for (uint32_t main : mains)
-    for (uint32_t qf = 1; qf <= 4; qf *= 2)
-      for (uint32_t qr = 1; qr <= 4; qr *= 2) {
+    for (uint32_t qf = 1; qf <= 2; qf *= 2)
+      for (uint32_t qr = 1; qr <= 2; qr *= 2) {
         const uint32_t nf = (full_blocks - main) * (kWaves / qf);
         const uint32_t nr = rest_blocks * div_up(rest_tiles, qr);
         if (nf + nr == 0) continue;
