@@ -1216,7 +1216,7 @@ uint32_t workgroups_per_xcd(const Geometry& g) {
 // FP6 and INT8 head-major rows have the same pitches.
 template <bool kFp6, bool kTm>
 hipError_t launch_self(Geometry g, uint32_t heads, hipStream_t stream) {
-  const SplitPlan plan = split_plan(g.tokens, g.rows, heads, device_cus());
+  const SplitPlan plan = split_plan(g.tokens, g.rows, heads, g.capacity, device_cus());
   g.q_blocks = (g.rows + kBlockQ - 1) / kBlockQ;
   g.total = g.q_blocks * heads;
   if (plan.split) {  // the first main_blocks full blocks here

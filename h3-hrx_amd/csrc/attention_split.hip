@@ -331,63 +331,79 @@ void k_attention_split(Args g) {
 
 inline uint32_t div_up(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-// The rule of split_plan prices a call in 64-key stages of k_attention_hm on a chip it does not
-// fill (1.25 us). Measured inside Stack::attend, right after the operands' kernels (S stages a
-// block, s stages a unit):
-//   k_attention_hm      up to one round of blocks 6.4 + 1.25 S us (10.7 us at S = 3, 12.3 at 4, 15.8
-//                       at 7, 26.3 at 16); 1.34 times that for each full round of one block per CU
-//                       (the engine clock falls); after full rounds, a last round that fills a share
-//                       f of the CUs takes about (1 + f) / 2 of a full one (its blocks start as CUs
-//                       free up, and run at a higher clock)
-//   k_attention_split   9 + 4 s us a round of units (10.9-13.1 us at s = 1, 16.9 at 2): its operands
-//                       come through each CU's L1 instead of being shared in LDS, about 20 bytes a
-//                       clock and CU
+// The rule of split_plan prices a call's ways of being divided in us, S stages of 64 keys a block. Fitted to
+// every way of 1,125 INT8 calls (1 to 24,000 tokens, 1 to 64 heads, all or some of the rows) behind their
+// operands' kernels in captured graphs, to 6.5 % in the root mean square; no call was measured slower than
+// undivided by it, in the FP6 form neither (175 calls).
+//   k_attention_hm      one block per CU, 5.75 + 1.14 S, to which a share f of the CUs at work adds 0.30 f^2
+//                       a stage (the engine clock falls) and 1.15 f in each of the first eight (every block
+//                       at once asks for operands just written); after full rounds a last round of share f
+//                       takes 0.67 + 0.32 f of one (its blocks start as CUs free up)
+//   k_attention_split   5.6 a round of units, 0.45 f in each of the first eight stages, and what its operands
+//                       take through the CU's L1: for each live tile and stage an eighth of 5.3 us where
+//                       V^T's rows are whole 128-byte lines apart (capacity % 64 == 0: the 32 rows of a load
+//                       then lie at the same place of their lines) and of 3.7 (1 + f / 4) where not (1,792
+//                       tokens of 4 heads: 25.4 against 21.5 us, 6,000 of 2: 133 against 105)
 // so 1,024 tokens of 8 heads take 16.5 us here against 26.3, and 8,193 of 16 heads, whose last round
-// would hold 16 blocks of one row each, 530 against 566; calls of up to seven stages, and from about
-// 3,000 keys on those that fill a quarter of the chip, are faster undivided.
-constexpr float kMainFixed = 5.1f, kMainFull = 1.34f, kSplitStage = 3.2f, kSplitFixed = 7.2f;
-constexpr float kSecondLaunch = 2.0f;
+// would hold 16 blocks of one row each, 530 against 566. 9,375 tokens of one head are faster undivided, 163
+// us against 198, and so are most calls of 3,000 keys that fill an eighth of the chip.
+constexpr float kMainFixed = 5.75f, kMainStage = 1.14f, kMainFull = 0.30f, kMainCold = 1.15f;
+constexpr float kMainLast = 0.67f, kMainLastShare = 0.32f;
+constexpr float kSplitFixed = 5.6f, kSplitCold = 0.45f;
+constexpr float kSplitAligned = 5.3f, kSplitStage = 3.7f, kSplitFull = 0.25f;
+constexpr float kSecondLaunch = 0.6f;
+constexpr uint32_t kColdStages = 8;
 
 // Time of `blocks` blocks of `stages` stages on k_attention_hm.
 float main_time(uint32_t blocks, uint32_t stages, uint32_t cus) {
-  const float block = stages + kMainFixed;
+  if (blocks == 0) return 0.0f;
   const uint32_t rounds = blocks / cus, extra = blocks % cus;
-  if (rounds == 0) return extra ? block : 0.0f;
-  return kMainFull * block * (rounds + (extra ? 0.5f + 0.5f * extra / cus : 0.0f));
+  const float share = (float)extra / cus;
+  auto round = [&](float f) { return kMainFixed + stages * (kMainStage + kMainFull * f * f); };
+  const float cold = kMainCold * std::min(stages, kColdStages);
+  if (rounds == 0) return cold * share + round(share);
+  return cold + round(1.0f) * (rounds + (extra ? kMainLast + kMainLastShare * share : 0.0f));
 }
 
-// The time after which `na` units of `da` each, then `nb` of `db`, have run on `cus` CUs in order.
+// The time after which `na` units of `da` each, then `nb` of `db`, have run on `cus` CUs in order: the
+// CUs that hold no unit of the last round of the first kind take the second kind's from then on.
 float makespan(uint32_t na, float da, uint32_t nb, float db, uint32_t cus) {
   const uint32_t rounds = na / cus, extra = na % cus;
-  const float early = rounds * da, late = (rounds + (extra ? 1 : 0)) * da;
-  if (nb == 0) return late;
-  // `cus - extra` CUs are free at `early`, the others at `late`
-  const uint32_t ahead = cus - extra;
-  const uint32_t lead = extra ? (uint32_t)(da / db) : 0u;  // units the early ones take before `late`
-  if (nb <= ahead * lead) return std::max(late, early + div_up(nb, ahead) * db);
-  const uint32_t left = nb - ahead * lead;
-  return std::max(late, early + lead * db) + div_up(left, cus) * db;
+  const float early = rounds * da, late = early + (extra ? da : 0.0f);
+  float end = late, next_early = early + db, next_late = late + db;
+  for (uint32_t left = nb; left > 0;) {
+    const bool from_early = extra == 0 || next_early <= next_late;
+    float& next = from_early ? next_early : next_late;
+    end = std::max(late, next);
+    next += db;
+    left -= std::min(left, from_early ? cus - extra : extra);
+  }
+  return end;
 }
 
 }  // namespace
 
-SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t cus) {
+SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t capacity, uint32_t cus) {
   const uint32_t stages = div_up(tokens, kKeys);
   const uint32_t full = rows / kBlockQ, rest_tiles = div_up(rows % kBlockQ, kTileQ);
   const uint32_t full_blocks = full * heads, rest_blocks = rest_tiles ? heads : 0u;
   SplitPlan best{false, 0, 0, 0};
-  // a split has to gain more than the model's error: 2 %, and a stage
-  const float whole = main_time(full_blocks + rest_blocks, stages, cus);
-  float best_time = std::min(0.98f * whole, whole - 1.0f);
   const uint32_t mains[2] = {full_blocks / cus * cus, full_blocks};
+  // a split has to gain more than the prices' error: 6 % of what follows the full rounds, which every way
+  // has, and a microsecond
+  const float whole = main_time(full_blocks + rest_blocks, stages, cus);
+  float best_time = whole - std::max(1.0f, 0.06f * (whole - main_time(mains[0], stages, cus)));
   for (uint32_t main : mains)
     for (uint32_t qf = 1; qf <= 2; qf *= 2)
       for (uint32_t qr = 1; qr <= 2; qr *= 2) {
         const uint32_t nf = (full_blocks - main) * (kWaves / qf);
         const uint32_t nr = rest_blocks * div_up(rest_tiles, qr);
         if (nf + nr == 0) continue;
-        const float df = div_up(stages, kWaves / qf) * kSplitStage + kSplitFixed;
-        const float dr = div_up(stages, kWaves / qr) * kSplitStage + kSplitFixed;
+        const float share = std::min(1.0f, (float)(nf + nr) / cus);
+        const float stage = capacity % 64 == 0 ? kSplitAligned : kSplitStage * (1.0f + kSplitFull * share);
+        const float fixed = kSplitFixed + kSplitCold * share * std::min(stages, kColdStages);
+        const float df = fixed + stage * stages * qf / kWaves;
+        const float dr = fixed + stage * stages * std::min(qr, rest_tiles) / kWaves;
         const float t = main_time(main, stages, cus) + (main ? kSecondLaunch : 0.0f) +
                         makespan(nf, df, nr, dr, cus);
         if (t < best_time) {

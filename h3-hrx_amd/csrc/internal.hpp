@@ -130,7 +130,8 @@ struct SplitPlan {
   bool split;
   uint32_t main_blocks, qw_full, qw_rest;
 };
-SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t cus);
+// `capacity`: the row pitch of V^T (halves), which the key-split kernel's loads depend on.
+SplitPlan split_plan(uint32_t tokens, uint32_t rows, uint32_t heads, uint32_t capacity, uint32_t cus);
 // Operands of k_attention_split in either layout: byte pitches of a token's code row and of a head
 // for K and Q, element pitches of a key's (query's) scale and of a head for the scales.
 struct SplitOperands {

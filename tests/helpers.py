@@ -189,3 +189,21 @@ def rank1_operands(rng, q_heads, q_tokens, q_cap, kv_heads, kv_tokens, kv_cap, c
     vt[:, :kv_tokens] = (rng.standard_normal((kv_heads * 128, kv_tokens), np.float32) *
                          0.3).astype(np.float16)
     return qc, qs, kc, ks, vt.view(np.uint16)
+
+
+# ---- the library's launch rules (host functions of libh3attn, internal.hpp)
+
+def split_plan(tokens, rows, heads, capacity, cus=256):
+    """How a self-attention call is divided: (main_blocks, qw_full, qw_rest), or None if it is not."""
+    import ctypes
+
+    import h3attn as H
+
+    class Plan(ctypes.Structure):
+        _fields_ = [("split", ctypes.c_bool), ("main_blocks", ctypes.c_uint32),
+                    ("qw_full", ctypes.c_uint32), ("qw_rest", ctypes.c_uint32)]
+
+    fn = H.lib()._ZN2h310split_planEjjjjj
+    fn.argtypes, fn.restype = [ctypes.c_uint32] * 5, Plan
+    p = fn(tokens, rows, heads, capacity, cus)
+    return (p.main_blocks, p.qw_full, p.qw_rest) if p.split else None
