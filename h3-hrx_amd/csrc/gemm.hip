@@ -25,6 +25,7 @@
 // What bounds it: at full occupancy the matrix cores' power (54 % busy at an engine clock of 1.5 GHz,
 // 31,104 tokens: 1.95-2.05 POP/s against torch._int_mm's 2.10); with one tile per CU or fewer, what a
 // CU can load (about 21 bytes a clock) and the latency of a step.
+#include <algorithm>
 #include <cmath>
 
 #include "internal.hpp"
@@ -456,6 +457,46 @@ hipError_t launch_few(Args g, hipStream_t stream) {
 
 }  // namespace
 
+// The tiling that prices lowest, in us, s steps of 128 bytes of K: fixed costs, what a tile costs besides its
+// steps (its fill and its epilogue, which nothing overlaps at one 256 x 256 tile per CU), and its steps.
+// n0, n1: 256 x 256 and 128 x 128 tiles per CU. 256 x 256 run one to a CU, in rounds; 128 x 128 on a ring
+// of two stages two to a CU; on a ring of four one, its loads four steps ahead. 64 x 128 where the others
+// leave three CUs of four idle. Past one round of 256 x 256 a smaller tile has to be 2 % cheaper, and 12 %
+// where A, W and the output are more than 200 MiB: it reads A and W more often, from HBM then, where the
+// 256 MB behind the L2s no longer holds what the launch touches. Fitted to 64 to 8,192 tokens at seven
+// (N, K); checked behind the quantizer with W from four buffers on 1,700 shapes of 33 to 64,000 tokens, 1 to
+// 56 heads, K 128 to 7,680: 3.7 % over the best tile in the mean, nearly all of it small calls that 64 x 128
+// would suit; 11 of them slower than on 256 x 256 by more than 1 %, by 6.7 % at most (without the rule for
+// 200 MiB 68, by 17 %). us on 256 x 256 / 128 x 128 ring 2 / ring 4, K 4,096, N 12,288: 129 tokens 57 / 29 /
+// 22, 513 64 / 41 / 44, 1,025 76 / 73 / 77, 5,000 246 / 279 / 298; 2,049 of K 1,024, N 21,504 113 / 87 / 108;
+// 641 of K 7,168, N 21,504 110 / 120 / 124; 34,453 of K 1,984, N 5,760 520 / 611 / 662.
+GemmTiling gemm_tiling(uint32_t m, uint32_t n, uint32_t k, uint32_t compute_units) {
+  if (m <= 32) return GemmTiling::kFew;
+  const float cus = compute_units, s = k / 128.0f;
+  auto tiles = [&](uint32_t bm, uint32_t bn) {
+    const uint32_t qk_width = n / 3 * 2;
+    const uint32_t qk = (qk_width + bn - 1) / bn, v = (n - qk_width + bn - 1) / bn;
+    return (m + bm - 1) / bm * (qk + v) / cus;
+  };
+  if (tiles(64, 128) <= 0.25f) return GemmTiling::k64x128;
+  const float n0 = tiles(256, 256), n1 = tiles(128, 128);
+  const float rounds = n0 <= 3.0f ? 0.84f * std::ceil(n0) + 0.16f * n0 : n0 + 0.2f;
+  const float t0 = n0 <= 1.0f ? 28.75f + s * (0.89f + 0.61f * n0)
+                              : 8.91f + rounds * (19.84f + 1.43f * s);
+  const float t2 = 7.01f + 3.43f * n1 +
+                   s * (n1 <= 2.0f   ? 0.64f + 0.29f * std::max(n1 - 1.0f, 0.0f)
+                        : n1 <= 4.0f ? 1.48f + 0.18f * (n1 - 2.0f)
+                                     : 0.21f + 0.475f * n1);
+  const float t4 = 7.6f + 4.95f * n1 +
+                   s * (n1 <= 1.0f   ? 0.35f
+                        : n1 <= 2.0f ? 0.85f
+                        : n1 <= 4.0f ? 1.17f + 0.36f * (n1 - 2.0f)
+                                     : 0.1f + 0.475f * n1);
+  const bool large = (float)m * k + (float)n * k + 2.0f * m * n >= 200.0f * 1048576.0f;
+  if (std::min(t2, t4) > (large ? 0.88f : n0 > 1.0f ? 0.98f : 1.0f) * t0) return GemmTiling::k256x256;
+  return t2 <= t4 ? GemmTiling::k128x128Ring2 : GemmTiling::k128x128Ring4;
+}
+
 hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_stride,
                               const int8_t* a, const int8_t* w, const float* ws, const float* as,
                               uint16_t* out, hipStream_t stream) {
@@ -471,38 +512,13 @@ hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_str
   g.k_stride = k_stride;
   g.qk_width = n / 3 * 2;
   g.cap = (m + kCapRows - 1) / kCapRows * kCapRows;
-  if (m <= 32) return launch_few(g, stream);
-  // The tile that prices lowest in us, s steps of 128 bytes of K: fixed costs, what a tile costs besides its
-  // steps (its fill and its epilogue, which nothing overlaps at one 256 x 256 tile per CU), and its steps.
-  // n0, n1: 256 x 256 and 128 x 128 tiles per CU. 256 x 256 run one to a CU, in rounds; 128 x 128 on a ring
-  // of two stages two to a CU; on a ring of four one, its loads four steps ahead. 64 x 128 where the others
-  // leave three CUs of four idle. Fitted to 64 to 8,192 tokens at (N, K) = (12,288, 4,096), (21,504, 7,168),
-  // (6,144, 2,048), (3,072, 5,120), (7,680, 3,072), (21,504, 1,024) and (15,360, 6,400), W in the caches and
-  // not: the choice costs 0.4 % over the best tile in the mean and 12 % at the most (prices per step of K
-  // alone: 2.9 and 47 %). Measured (us: 256 x 256 / 128 x 128 ring 2 / ring 4), at K = 4,096, N = 12,288:
-  // 129 tokens 57 / 29 / 22, 513 64 / 41 / 44, 1,025 76 / 73 / 77, 5,000 246 / 279 / 298; 2,049 at K =
-  // 1,024, N = 21,504 113 / 87 / 108; 641 at K = 7,168, N = 21,504 110 / 120 / 124.
-  const float cus = device_cus(), s = k / 128.0f;
-  auto tiles = [&](uint32_t bm, uint32_t bn) {
-    const uint32_t qk = (g.qk_width + bn - 1) / bn, v = (n - g.qk_width + bn - 1) / bn;
-    return (m + bm - 1) / bm * (qk + v) / cus;
-  };
-  if (tiles(64, 128) <= 0.25f) return launch_tiles<1, 1, 4>(g, stream);
-  const float n0 = tiles(256, 256), n1 = tiles(128, 128);
-  const float rounds = n0 <= 3.0f ? 0.84f * std::ceil(n0) + 0.16f * n0 : n0 + 0.2f;
-  const float t0 = n0 <= 1.0f ? 28.75f + s * (0.89f + 0.61f * n0)
-                              : 8.91f + rounds * (19.84f + 1.43f * s);
-  const float t2 = 7.01f + 3.43f * n1 +
-                   s * (n1 <= 2.0f   ? 0.64f + 0.29f * std::max(n1 - 1.0f, 0.0f)
-                        : n1 <= 4.0f ? 1.48f + 0.18f * (n1 - 2.0f)
-                                     : 0.21f + 0.475f * n1);
-  const float t4 = 7.6f + 4.95f * n1 +
-                   s * (n1 <= 1.0f   ? 0.35f
-                        : n1 <= 2.0f ? 0.85f
-                        : n1 <= 4.0f ? 1.17f + 0.36f * (n1 - 2.0f)
-                                     : 0.1f + 0.475f * n1);
-  if (t0 <= t2 && t0 <= t4) return launch_tiles<4, 2, 2>(g, stream);
-  return t2 <= t4 ? launch_tiles<2, 1, 2>(g, stream) : launch_tiles<2, 1, 4>(g, stream);
+  switch (gemm_tiling(m, n, k, device_cus())) {
+    case GemmTiling::kFew: return launch_few(g, stream);
+    case GemmTiling::k64x128: return launch_tiles<1, 1, 4>(g, stream);
+    case GemmTiling::k128x128Ring4: return launch_tiles<2, 1, 4>(g, stream);
+    case GemmTiling::k128x128Ring2: return launch_tiles<2, 1, 2>(g, stream);
+    default: return launch_tiles<4, 2, 2>(g, stream);
+  }
 }
 
 }  // namespace h3

@@ -92,6 +92,9 @@ hipError_t launch_prepare_qk_rope_mean(const h3_prepare_cfg& cfg, uint32_t token
 hipError_t launch_transpose(uint32_t width, uint32_t row_capacity, uint32_t row_stride,
                             uint32_t col_offset, uint32_t elem, uint32_t tile, uint32_t launch_rows,
                             uint32_t rows, const void* x, uint16_t* out, hipStream_t stream);
+// The tiling of an INT8 projection of m tokens, n channels and K = k (gemm.hip).
+enum class GemmTiling : uint32_t { kFew, k64x128, k128x128Ring4, k128x128Ring2, k256x256 };
+GemmTiling gemm_tiling(uint32_t m, uint32_t n, uint32_t k, uint32_t cus);
 hipError_t launch_gemm_i8_qkv(uint32_t m, uint32_t n, uint32_t k, uint32_t k_stride,
                               const int8_t* a, const int8_t* w, const float* ws, const float* as,
                               uint16_t* out, hipStream_t stream);

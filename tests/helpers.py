@@ -207,3 +207,17 @@ def split_plan(tokens, rows, heads, capacity, cus=256):
     fn.argtypes, fn.restype = [ctypes.c_uint32] * 5, Plan
     p = fn(tokens, rows, heads, capacity, cus)
     return (p.main_blocks, p.qw_full, p.qw_rest) if p.split else None
+
+
+GEMM_TILINGS = ("few", "64x128", "128x128 ring 4", "128x128 ring 2", "256x256")
+
+
+def gemm_tiling(m, n, k, cus=256):
+    """The tiling of an INT8 projection of m tokens, n channels and K = k, one of GEMM_TILINGS."""
+    import ctypes
+
+    import h3attn as H
+
+    fn = H.lib()._ZN2h311gemm_tilingEjjjj
+    fn.argtypes, fn.restype = [ctypes.c_uint32] * 4, ctypes.c_uint32
+    return GEMM_TILINGS[fn(m, n, k, cus)]
