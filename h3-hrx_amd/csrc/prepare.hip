@@ -701,8 +701,8 @@ __device__ __forceinline__ void unpack8(uint4 b, uint32_t elem, float (&v)[8]) {
 
 // kRope false: the column mean of x itself (h3_colmean_f32), 16 adjacent columns per workgroup; the
 // producers only widen, and weight, the tables and r_in are not read. One lane per column with 16
-// loads in flight was bound by their latency, 34 ns a row against the chain's 3.54: 86 -> 26 us at
-// 2,501 x 7,168, 5,660 -> 730 us at 129,024 x 4,096.
+// loads in flight was bound by their latency, 34 ns a row against the chain's 3.54: 86 -> 18 us at
+// 2,501 x 7,168, 5,660 -> 550 us at 129,024 x 4,096.
 template <bool kRope>
 __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
     const void* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ cos_t,
@@ -781,6 +781,28 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
 
   float acc = 0.0f;
   const int lane = threadIdx.x;  // the chain lanes (wave 0, lanes 0-15)
+  // acc plus `groups` groups of 32 tokens of a column, the next group's values read under the adds.
+  auto add_groups = [&](const float* col, auto groups) __attribute__((always_inline)) {
+    float4 cur[8], nxt[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cur[i] = *reinterpret_cast<const float4*>(col + 4 * i);
+    for (uint32_t g = 0; g < groups; ++g) {
+      if (g + 1 < groups) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          nxt[i] = *reinterpret_cast<const float4*>(col + 32 * (g + 1) + 4 * i);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        acc = acc + cur[i].x;
+        acc = acc + cur[i].y;
+        acc = acc + cur[i].z;
+        acc = acc + cur[i].w;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
+    }
+  };
   // One chunk: producers store chunk j + 1 and load chunk j + 3 into the ring slot chunk j
   // left; lanes 0-15 add chunk j. Slot indices are compile-time (the loop is unrolled by kRing).
   auto chunk = [&](uint32_t j, auto slot) {
@@ -792,28 +814,13 @@ __global__ __launch_bounds__(kColmeanThreads) void k_rope_colmean(
     if (threadIdx.x < kSlab) {
       const float* col = tile[j & 1][lane];
       const uint32_t n = min((uint32_t)kChunk, tokens - j * kChunk);
+      // A whole chunk's groups are a compile-time count, so that the groups' registers alternate: with a
+      // run-time count each add is followed by a copy (17,537 tokens x 36 heads 237 -> 263 us).
       const uint32_t groups = n / 32;
-      if (groups > 0) {
-        float4 cur[8], nxt[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) cur[i] = *reinterpret_cast<const float4*>(col + 4 * i);
-        for (uint32_t g = 0; g < groups; ++g) {
-          if (g + 1 < groups) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              nxt[i] = *reinterpret_cast<const float4*>(col + 32 * (g + 1) + 4 * i);
-          }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            acc = acc + cur[i].x;
-            acc = acc + cur[i].y;
-            acc = acc + cur[i].z;
-            acc = acc + cur[i].w;
-          }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
-        }
-      }
+      if (n == kChunk)
+        add_groups(col, std::integral_constant<uint32_t, kChunk / 32>{});
+      else if (groups > 0)
+        add_groups(col, groups);
       for (uint32_t i = 32 * groups; i < n; ++i) acc = acc + col[i];
     }
     __syncthreads();
