@@ -182,15 +182,16 @@ hipError_t launch_attention_cross(const h3_cross_cfg& cfg, const int32_t* qi, co
                                   const uint8_t* key_mask, uint16_t* out, hipStream_t stream);
 // The query cubes [0, cubes) of every head whose routes keep (nearly) every key cube, the VSA
 // runtime's prefix: their own launches, each cube split into `splits` ranges of the key cubes when
-// `splits` > 1, with the ranges' partial results in `part` (vsa_part_bytes). Empty: no such cubes.
+// `splits` > 1, with the ranges' partial results in `part` (vsa_part_bytes). No cubes: one order for all.
 // `kept`: about how many key cubes each other query cube keeps (0: unknown).
 struct VsaPrefix {
   uint32_t cubes = 0, splits = 1, kept = 0;
   float* part = nullptr;
 };
-// The number of ranges for `cubes` prefix cubes of `heads` heads over `blocks` key cubes, and the
-// bytes of their partial results (0 for one range).
-size_t vsa_part_bytes(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t* splits);
+// How a runtime of `heads` heads over `blocks` key cubes, `cubes` of them prefix, launches its attention
+// (part not set), and the bytes of its ranges' partial results (0 for one range: at most 34 MB).
+VsaPrefix vsa_prefix(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t topk, uint32_t cus);
+size_t vsa_part_bytes(uint32_t heads, const VsaPrefix& prefix);
 // The int8 token-major attention over the cubes `routes` keeps (attention.hip). With a
 // `workspace` of scales_workspace_bytes(cfg) bytes the key scales are first transposed into it
 // (head-major) and the kernel reads them from there; with nullptr it reads the token-major

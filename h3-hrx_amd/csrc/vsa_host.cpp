@@ -254,10 +254,8 @@ int h3_vsa_build_bits(const int32_t* src, const int32_t* inverse, const int32_t*
       return st;
     }
   }
-  r->prefix.cubes = prefix_blocks;
-  r->prefix.kept = prefix_blocks + r->cfg.topk + 2;  // the prefix, its own choice, an edge or two
-  const size_t part_bytes = vsa_part_bytes(heads, prefix_blocks, blocks, &r->prefix.splits);
-  if (part_bytes) {
+  r->prefix = vsa_prefix(heads, prefix_blocks, blocks, r->cfg.topk, device_cus());
+  if (const size_t part_bytes = vsa_part_bytes(heads, r->prefix)) {
     if ((st = allocate(&r->part, part_bytes))) {
       release(r);
       delete r;

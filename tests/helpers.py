@@ -221,3 +221,19 @@ def gemm_tiling(m, n, k, cus=256):
     fn = H.lib()._ZN2h311gemm_tilingEjjjj
     fn.argtypes, fn.restype = [ctypes.c_uint32] * 4, ctypes.c_uint32
     return GEMM_TILINGS[fn(m, n, k, cus)]
+
+
+def vsa_prefix(heads, cubes, blocks, topk, cus=256):
+    """(cubes, splits) of the query cubes the VSA runtime launches apart, (0, 1) for one order for all."""
+    import ctypes
+
+    import h3attn as H
+
+    class Prefix(ctypes.Structure):
+        _fields_ = [("cubes", ctypes.c_uint32), ("splits", ctypes.c_uint32),
+                    ("kept", ctypes.c_uint32), ("part", ctypes.c_void_p)]
+
+    fn = H.lib()._ZN2h310vsa_prefixEjjjjj
+    fn.argtypes, fn.restype = [ctypes.c_uint32] * 5, Prefix
+    p = fn(heads, cubes, blocks, topk, cus)
+    return p.cubes, p.splits
