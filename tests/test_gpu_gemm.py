@@ -13,7 +13,7 @@ import pytest
 
 import h3attn as H
 import oracle as O
-from helpers import from_dev, to_dev
+from helpers import from_dev, gemm_tiling, to_dev
 from test_oracle_gemm import reference_inputs, same_bits
 
 pytestmark = pytest.mark.gpu
@@ -58,7 +58,7 @@ def test_compact_qkv_across_the_row_bound(dev, rows):
 
 def test_compact_qkv_half_step_and_row_padding(dev):
     """K = 192 (one full 128-byte step and a 64-byte one), rows padded to 256 bytes with
-    garbage past K, N = 1152 (a partial last V tile), M = 700."""
+    garbage past K, N = 1152, M = 700 (a partial last tile of tokens)."""
     rng = np.random.default_rng(3)
     m, n, k, stride = 700, 1152, 192, 256
     a = rng.integers(-128, 128, (m, stride), dtype=np.int8)
@@ -71,9 +71,10 @@ def test_compact_qkv_half_step_and_row_padding(dev):
 
 @pytest.mark.parametrize("k", [256, 320, 384, 448, 576])
 def test_compact_qkv_step_counts(dev, k):
-    """K advances 128 bytes a step through two LDS stages: 256-576 bytes are even and odd step
-    counts (2-5), with and without a final 64-byte half step (320, 448, 576), rows padded past K
-    by garbage and a partial last tile in M and in V, bit-exact."""
+    """64 x 128 tiles, K 128 bytes a step through four LDS stages: 256-576 bytes are step counts below,
+    at and past the ring (2-5), with and without a final 64-byte half step (320, 448, 576), rows padded
+    past K by garbage and a partial last tile in M, bit-exact."""
+    assert gemm_tiling(300, 768, k) == "64x128"
     rng = np.random.default_rng(k)
     m, n, stride = 300, 768, k + 64
     a = rng.integers(-128, 128, (m, stride), dtype=np.int8)
@@ -120,13 +121,7 @@ def test_dit_projection_shape_on_sampled_tokens(dev, m):
     assert np.all(vt[:, m:] == 0)
 
 
-# (tokens, channels) of every way the projection is tiled (32-token workgroups, 64 x 128, 128 x 128
-# on four and on two ring stages at full and partial last tiles, 256 x 256), with step counts below,
-# at and past the rings' lengths and a 64-byte K tail
-@pytest.mark.parametrize("k", [64, 128, 192, 384, 512, 704])
-@pytest.mark.parametrize("tokens,n", [(1, 384), (32, 1152), (33, 384), (100, 8448), (200, 21504),
-                                      (520, 12288), (1100, 21504), (1500, 21504)])
-def test_every_tiling_is_bit_exact(dev, tokens, n, k):
+def check_against_exact_sums(dev, tokens, n, k):
     import torch
 
     g = torch.Generator(device=dev).manual_seed(tokens + n + k)
@@ -137,10 +132,10 @@ def test_every_tiling_is_bit_exact(dev, tokens, n, k):
     scales = (torch.rand(tokens, generator=g, device=dev) + 0.5) * 1e-3
     out = torch.full((H.compact_qkv_elements(tokens, n) + 64,), float("nan"), dtype=torch.float16,
                      device=dev)
-    print(f"gemm tiling tokens={tokens} n={n} k={k}", flush=True)
+    print(f"gemm tiling tokens={tokens} n={n} k={k} {gemm_tiling(tokens, n, k)}", flush=True)
     H.gemm_i8_qkv_256(H.GemmCfg(k, n, stride, 4), tokens, a, w, ws, scales, out[:-64])
     acc = a[:, :k].double() @ w[:, :k].double().t()  # exact: below 2^53
-    v = (acc.float() * ws) * scales[:, None] + 0.0   # |acc| < 2^24: exact in f32 as in the kernel
+    v = (acc.float() * ws) * scales[:, None] + 0.0   # int32 to f32 rounds to nearest, as the kernel's does
     v = v.clamp(-65472.0, 65472.0).half()
     cap, two = -(-tokens // 256) * 256, 2 * n // 3
     vt = torch.zeros((n - two, cap), dtype=torch.float16, device=dev)
@@ -150,9 +145,35 @@ def test_every_tiling_is_bit_exact(dev, tokens, n, k):
     assert torch.isnan(out[-64:]).all(), "written past the output"
 
 
-# long K, where the prices per step decide: 256 x 256 in one round and in two, 128 x 128 on four stages with
-# the capacity's last columns past the tokens' tiles and inside them, 128 x 128 on two stages
-@pytest.mark.parametrize("tokens,n,k", [(520, 21504, 6208), (1100, 21504, 7232), (257, 21504, 7232),
-                                        (900, 3072, 5184), (300, 12288, 4160)])
-def test_tilings_of_a_long_k_are_bit_exact(dev, tokens, n, k):
-    test_every_tiling_is_bit_exact(dev, tokens, n, k)
+# (tokens, channels) of the ways a short K is tiled (32-token workgroups, 64 x 128, 128 x 128 on two ring
+# stages and from K = 512 on four, at full and partial last tiles), with step counts below, at and past
+# the rings' lengths and a 64-byte K tail
+@pytest.mark.parametrize("k", [64, 128, 192, 384, 512, 704])
+@pytest.mark.parametrize("tokens,n,tiling", [
+    (1, 384, "few"), (32, 1152, "few"), (33, 384, "64x128"), (100, 8448, None),
+    (200, 21504, "128x128 ring 2"), (520, 12288, "128x128 ring 2"), (1100, 21504, "128x128 ring 2"),
+    (1500, 21504, "128x128 ring 2")])
+def test_every_tiling_of_a_short_k_is_bit_exact(dev, tokens, n, tiling, k):
+    tiling = tiling or f"128x128 ring {4 if k >= 512 else 2}"
+    assert gemm_tiling(tokens, n, k) == tiling
+    check_against_exact_sums(dev, tokens, n, k)
+
+
+# long K: 256 x 256 in one round, 128 x 128 on four stages with the capacity's last columns past the
+# tokens' tiles and inside them, 128 x 128 on two stages in several rounds
+@pytest.mark.parametrize("tokens,n,k,tiling", [
+    (520, 21504, 6208, "256x256"), (1100, 21504, 7232, "256x256"), (257, 21504, 7232, "128x128 ring 4"),
+    (900, 3072, 5184, "128x128 ring 4"), (300, 12288, 4160, "128x128 ring 2")])
+def test_tilings_of_a_long_k_are_bit_exact(dev, tokens, n, k, tiling):
+    assert gemm_tiling(tokens, n, k) == tiling
+    check_against_exact_sums(dev, tokens, n, k)
+
+
+# 256 x 256 with a partial last tile of tokens and, the heads odd, of V, in one round and in three, at
+# even and odd step counts with and without a 64-byte K tail (the rule takes it from about 15 steps on)
+@pytest.mark.parametrize("tokens,n,k", [
+    (700, 384 * 55, 3264), (700, 384 * 55, 3328), (700, 384 * 55, 3392), (700, 384 * 55, 3456),
+    (3000, 384 * 41, 1984), (3000, 384 * 41, 2048), (3000, 384 * 41, 2112), (3000, 384 * 41, 2176)])
+def test_256_tiles_with_partial_edges_are_bit_exact(dev, tokens, n, k):
+    assert gemm_tiling(tokens, n, k) == "256x256"
+    check_against_exact_sums(dev, tokens, n, k)
