@@ -1,28 +1,51 @@
 """Attention calls whose query blocks do not fill the chip, or leave a partial last round, run (in
 part) on the key-split kernel: the ways a call is divided, at the edges of its tiles and units,
-against the f64 oracle at the head-major suite's bar (1e-3 + 2e-3 rel), in every operand layout the
-dispatch accepts. Both layouts divide a call alike and the kernel reads them through pitches, so
-their outputs agree bit for bit."""
+against the f64 oracle at the head-major suite's bar (1e-3 + 2e-3 rel) in both INT8 layouts, and in the
+FP6 form at its suite's. Both layouts divide a call alike and the kernel reads them through pitches, so
+their outputs agree bit for bit. Every case asserts how the rule divides it."""
 import numpy as np
 import pytest
 
 import h3attn as H
 import oracle as O
-from helpers import filled, head_major_operands, pack_codes, to_dev
+from helpers import (filled, from_dev, head_major_operands, north_star_ok, pack_codes, split_plan,
+                     to_dev)
+from test_gpu_fp6 import operands, oracle_rows, run_fp6
+from test_gpu_i4 import pack_i4
 
 pytestmark = pytest.mark.gpu
 
 
-# (tokens, token_count, query heads, key/value heads, pad): fewer stages than key groups; one row,
-# one key past a stage, a wave with no live row; every number of tiles in a last block; a chip-filling
-# count of full blocks with a partial one left over; head wrap and padded output pitches
-@pytest.mark.parametrize("tokens,count,q_heads,kv_heads,pad", [
-    (1, 1, 2, 2, 0), (33, 33, 3, 3, 128), (65, 65, 2, 2, 0), (129, 129, 56, 56, 0),
-    (257, 256, 8, 8, 0), (512, 449, 4, 2, 128), (1000, 1000, 7, 7, 0), (1024, 1024, 8, 8, 128),
-    (2047, 2047, 8, 8, 0), (4160, 300, 5, 5, 0), (8193, 8193, 16, 16, 0)])
-def test_divided_calls_match_the_oracle_in_both_layouts(dev, tokens, count, q_heads, kv_heads, pad):
+# (tokens, token_count, query heads, key/value heads, pad) and the division, None for undivided or (blocks on
+# the undivided kernel, tiles per unit of the other full blocks, of the last, partial blocks): single calls
+# of one stage; two, three and seven stages (idle key groups); one key past eight stages; one to eight
+# live tiles in the last block; only whole blocks; a wave with no live row; units of two tiles; whole
+# rounds with the partial blocks, with a round of full blocks, and with both left over; head wrap and
+# padded output pitches
+CASES = [
+    (1, 1, 2, 2, 0, None), (33, 33, 3, 3, 128, None),
+    (65, 65, 2, 2, 0, (0, 1, 1)), (129, 129, 5, 5, 128, (0, 1, 1)), (257, 256, 8, 8, 0, (0, 1, 1)),
+    (385, 385, 2, 2, 0, (0, 1, 1)), (447, 447, 3, 3, 0, (0, 1, 1)), (448, 448, 5, 5, 0, (0, 1, 1)),
+    (449, 449, 3, 3, 0, (0, 1, 1)), (512, 449, 4, 2, 128, (0, 1, 1)), (513, 513, 4, 4, 0, (0, 1, 1)),
+    (577, 545, 4, 4, 0, (0, 1, 1)), (640, 609, 2, 2, 128, (0, 1, 1)), (200, 161, 4, 4, 0, (0, 1, 1)),
+    (1000, 1000, 7, 7, 0, (0, 1, 1)), (1024, 1024, 8, 8, 128, (0, 1, 1)),
+    (2047, 2047, 8, 8, 0, None), (4160, 300, 5, 5, 0, (0, 1, 1)), (2816, 2816, 3, 3, 0, (0, 2, 1)),
+    (2806, 2806, 3, 3, 0, (0, 2, 2)), (4858, 184, 50, 50, 0, (0, 1, 2)),
+    (4864, 4864, 14, 14, 0, (256, 1, 1)), (8193, 8193, 16, 16, 0, (512, 1, 1)),
+    (34007, 34007, 2, 2, 0, (256, 1, 1))]
+
+
+def check_division(tokens, count, heads, plan):
+    got = split_plan(tokens, count, heads, H.capacity(tokens))
+    assert got == plan, got
+
+
+@pytest.mark.parametrize("tokens,count,q_heads,kv_heads,pad,plan", CASES)
+def test_divided_calls_match_the_oracle_in_both_layouts(dev, tokens, count, q_heads, kv_heads, pad,
+                                                        plan):
     import torch
 
+    check_division(tokens, count, q_heads, plan)
     cap = O.capacity(tokens)
     rng = np.random.default_rng(tokens + 13 * q_heads)
     qc, qs, _, _, _ = head_major_operands(rng, q_heads, tokens, cap, late_match=False)
@@ -64,3 +87,29 @@ def test_divided_calls_match_the_oracle_in_both_layouts(dev, tokens, count, q_he
                            vt[:touched * 128], tokens, cap, touched, rows)
     err = np.abs(values.reshape(count, touched, 128)[rows] - want)
     assert np.all(err <= 1e-3 + 2e-3 * np.abs(want)), float(err.max())
+
+
+@pytest.mark.parametrize("tokens,count,heads,plan", [
+    (c[0], c[1], c[2], c[5]) for c in CASES if c[2] == c[3] and c[4] == 0 and c[5] and c[0] < 10000])
+def test_divided_fp6_calls_match_the_oracle(dev, tokens, count, heads, plan):
+    import torch
+
+    check_division(tokens, count, heads, plan)
+    cap = H.capacity(tokens)
+    rng = np.random.default_rng(tokens + 31 * heads)
+    q, k, qs, ks, vt = operands(rng, tokens, heads, cap)
+    print(f"divided FP6 call: S={tokens} rows={count} heads={heads}", flush=True)
+    got, _, cfg = run_fp6(dev, q, qs, k, ks, vt, tokens, cap, heads, token_count=count)
+    a6 = got.view(np.float16).astype(np.float64)
+    assert np.isfinite(a6).all()
+    rows = np.unique(np.concatenate([[0, min(31, count - 1), count - 1],
+                                     rng.integers(0, count, 5)])).astype(np.int32)
+    want = oracle_rows(q, qs, k, ks, vt, tokens, cap, heads, rows)
+    mx, mean = north_star_ok(a6.reshape(count, heads, 128)[rows], want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+    # every row against the int8-MFMA int4 kernel, which divides no call
+    out4 = torch.zeros((count, heads * 128), dtype=torch.float16, device=dev)
+    H.attention_i4qk(cfg, count, heads, to_dev(pack_i4(q), dev), to_dev(qs, dev),
+                     to_dev(pack_i4(k), dev), to_dev(ks, dev), to_dev(vt, dev), out4)
+    a4 = from_dev(out4).view(np.float16).astype(np.float64)
+    assert np.all(np.abs(a6 - a4) <= 2e-3 + 4e-3 * np.abs(a4))
