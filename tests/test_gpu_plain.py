@@ -115,3 +115,34 @@ def test_attention_output_shape_on_sampled_rows(dev, tokens):
     assert np.array_equal(got_c, wc)
     assert np.array_equal(got_s.view(np.uint32), ws.view(np.uint32))
     assert np.all(np.isfinite(scales.cpu().numpy()))
+
+
+# 16-bit rows of up to 4,096 channels: a wave walks ceil(tokens / (8 CUs)) rows, at most eight, the next row's
+# loads under the current one's work. Two to eight rows with ragged ends and idle lanes (width 768), every
+# row against the same rows in calls of one row per wave (which the tests above hold to the oracle).
+@pytest.mark.parametrize("tokens", [2049, 4097, 5000, 8192, 14335, 14337, 16385, 20000])
+@pytest.mark.parametrize("width", [256, 768, 4096])
+@pytest.mark.parametrize("elem", [H.H3_ELEM_F16, H.H3_ELEM_BF16])
+def test_walks_of_several_rows_give_the_single_rows_codes(dev, tokens, width, elem):
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(tokens + width)
+    x = torch.randn((tokens, width), generator=g, device=dev) * 3
+    x = x.to(torch.float16 if elem == H.H3_ELEM_F16 else torch.bfloat16)
+    x[5, 1], x[tokens - 1, 0] = float("nan"), float("inf")
+    stride = width + 64
+    cfg = H.PreparePlainCfg(width, 256, stride, elem)
+    single = 8 * torch.cuda.get_device_properties(dev).multi_processor_count
+    print(f"prepare_plain walk tokens={tokens} width={width} elem={elem}", flush=True)
+
+    def run(step):
+        codes = torch.full((tokens, stride), 0x55, dtype=torch.int8, device=dev)
+        scales = torch.full((tokens,), 7.0, device=dev)
+        for r in range(0, tokens, step):
+            n = min(step, tokens - r)
+            H.prepare_plain_i8(cfg, n, x[r:r + n], codes[r:r + n], scales[r:r + n])
+        torch.cuda.synchronize()
+        return codes, scales.view(torch.int32)
+
+    (got_c, got_s), (want_c, want_s) = run(tokens), run(single)
+    assert torch.equal(got_c, want_c) and torch.equal(got_s, want_s)
