@@ -1001,15 +1001,16 @@ __global__ __launch_bounds__(256) void k_prepare_fused(FusedArgs a) {
 
 inline uint32_t div_up(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-// Heads per workgroup of the RoPE quantizer. One workgroup per 32 tokens walking all heads leaves a
-// short sequence's launch with few workgroups and a long serial walk: at 4,097 tokens x 56 heads (129
-// workgroups) 74 us, in chunks of 8 heads 33 us; 8,193 x 16 34 -> 23 (chunks of 4); 31,104 x 32 116 ->
-// 109. From 65,536 tokens on whole walks are as fast (129,024 x 32: 417 against 420 us) and read the
-// tables once.
-uint32_t rope_chunk(uint32_t tokens, uint32_t heads) {
+// Heads per workgroup of the RoPE quantizer in a launch of `operands` operands (2: Q and K together). One
+// workgroup per 32 tokens walking all heads leaves a short sequence's launch with few workgroups and a long
+// serial walk: at 4,097 tokens x 56 heads (129 workgroups) 72 us, in chunks of 4 or 8 heads 32; 8,193 x 16 32 ->
+// 22 (chunks of 4); 31,104 x 32 116 -> 110. Q, K and V^T together, 4,097 x 56: 105 us, 81 in chunks of 4, 77
+// of 8; 4,097 x 8: 19 of 8, 16 of 4. From 65,536 tokens on whole walks are as fast (129,024 x 32: 417 against
+// 420 us) and read the tables once.
+uint32_t rope_chunk(uint32_t tokens, uint32_t heads, uint32_t operands) {
   const uint32_t blocks = div_up(tokens, kRopeGroups);
   if (blocks >= 8 * device_cus()) return div_up(heads, kRowsAhead) * kRowsAhead;
-  return blocks * div_up(heads, 8) < 4 * device_cus() ? 4 : 8;
+  return operands * blocks * div_up(heads, 8) < 4 * device_cus() ? 4 : 8;
 }
 
 }  // namespace
@@ -1089,7 +1090,7 @@ hipError_t launch_prepare_fused(const h3_prepare_cfg& q, const h3_prepare_cfg& k
   a.extra_q = q.extra_scale;
   a.extra_k = k.extra_scale;
   a.eps = q.eps;
-  a.chunk = rope_chunk(tokens, q.heads);
+  a.chunk = rope_chunk(tokens, q.heads, 2);
   a.token_blocks = div_up(tokens, kRopeGroups);
   a.rows = a.token_blocks * div_up(q.heads, a.chunk);
   a.width = t.width;
@@ -1160,7 +1161,7 @@ hipError_t launch_prepare_qk_rope_mean(const h3_prepare_cfg& cfg, uint32_t token
                                        const float* weight, const float* cos_t,
                                        const float* sin_t, const float* mean, int32_t* codes,
                                        float* scales, hipStream_t stream) {
-  const uint32_t chunk = rope_chunk(tokens, cfg.heads);
+  const uint32_t chunk = rope_chunk(tokens, cfg.heads, 1);
   const dim3 grid(div_up(tokens, kRopeGroups), div_up(cfg.heads, chunk));
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, weight, cos_t, sin_t, mean, codes,
