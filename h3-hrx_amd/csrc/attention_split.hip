@@ -1,12 +1,16 @@
 // INT8-QK / f16-PV attention for the query blocks that would leave most of the chip idle: the whole
-// call of a short sequence, and the last, partial round of a longer one. The operands, the
-// arithmetic and the results' tolerance are those of k_attention_hm (attention_hm.hip); what
-// differs is who does the work.
+// call of a short sequence, and the last, partial round of a longer one. The operands, the result and its
+// tolerance are those of k_attention_hm (attention_hm.hip); what differs is who does the work, and the
+// last bits: each group of keys has its own running max, the scores are multiplied by their scales
+// directly (there by one FMA that also takes out the accumulators' bias), and the row sum adds the
+// probabilities in f32 before they are rounded to f16 for PV (there the rounded ones). A call's rows can
+// come from both kernels, so a row's last bits depend on how its call is divided. Against 64 bits, 1,024
+// tokens of 8 heads: 2.9e-4 of the result here, 3.0e-4 there.
 //
 // k_attention_hm gives 256 queries of one head to a workgroup, which walks every key: a call of B
 // blocks takes ceil(B / CUs) rounds of a whole walk, however few blocks the last round holds. Here
-// a workgroup's eight waves are QW (one or two) tiles of 32 queries times KS = 8 / QW groups of keys: group g
-// walks the 64-key stages g, g + KS, ..., each wave with an online softmax of its own, and the KS
+// a workgroup's eight waves are QW (one or two) tiles of 32 queries times KS = 8 / QW groups of keys:
+// group g walks the 64-key stages g, g + KS, ..., each wave with an online softmax of its own, and the KS
 // partial results of a tile are combined through LDS at the end. A block's work is then spread
 // over 8 / QW workgroups, each of which takes 1 / KS of the walk, without device memory for the
 // partial results.
