@@ -39,7 +39,8 @@ struct h3_stack {
   h3_prepare_cfg prep_q{}, prep_k{};
   h3_attention_cfg attention{};
   h3_transpose_cfg transpose{};
-  // IntQk (src/stack.rs:229-238)
+  // IntQk (src/stack.rs:229-238). zmean: the reference's zero mean, handed out with the others; the
+  // kernels here take no mean instead.
   h3_view qi{}, ki{}, qs{}, ks{}, kmean{}, zmean{}, vt{};
   // The fused route's three independent prepare launches run as branches (the reference
   // records prep_q, prep_k and the V transpose as separate graph branches joined before the

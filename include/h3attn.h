@@ -524,7 +524,9 @@ typedef struct h3_vsa h3_vsa;
 /* Runtime::new (src/vsa/device.rs:49-188) for the INT8 attention (bits 8): uploads the plan
  * (HOST arrays as h3_vsa_plan fills them), derives the h3.vsa.* and attention configs, and
  * allocates the gathered q/k/v, block means, scores, routes, operand and output buffers and
- * one zeroed K-mean vector per layer. The only allocating VSA call. */
+ * one zeroed K-mean vector per layer, and, with a prefix whose cubes are split over the key cubes, their
+ * partial results: 33 KB a range, at most one generation of them (1,024, 34 MB, on 256 compute
+ * units). All of it is held until h3_vsa_destroy. The only allocating VSA call. */
 int h3_vsa_build(const int32_t *src, const int32_t *inverse, const int32_t *lengths,
                  uint32_t blocks, uint32_t seq_len, uint32_t prefix_blocks,
                  const h3_vsa_options *options, uint32_t heads, uint32_t layers, h3_vsa **out);
