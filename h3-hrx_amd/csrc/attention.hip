@@ -1736,10 +1736,10 @@ static uint32_t vsa_generation() { return std::max(1u, 4u * device_cus()); }
 // all `blocks` of them. A walk of L cubes takes about 0.4 L us with one workgroup per CU and L us in a full
 // generation; the launches and the combination take 10 us. One order for all cubes walks the whole list in
 // every generation, `kept` of it at that generation's share of the chip and the rest with the prefix's items
-// alone; apart, the prefix's ranges come first and every generation ends at `kept`. Of 260 runtime calls
-// timed both ways (29 to 811 key cubes, 1 to 40 heads, keep 2 to 99 %) seven take the slower way, by 11 % at
-// most (306 against 339 us); always apart 64 did, by 26 % (112 cubes of 18 heads, 28 of them prefix, all
-// kept: 562 us in one order, 703 apart).
+// alone; apart, the prefix's ranges come first and every generation ends at `kept`. Of 560 runtime calls
+// timed both ways (13 to 923 key cubes, 1 to 40 heads, keep 2 to 99 %) 33 take the way that is slower by more
+// than 2 %, by 18 % at most (87 cubes of 16 heads, 21 of them prefix: 242 against 285 us); always apart 213 did,
+// by 48 % at most (112 cubes of 18 heads, 28 of them prefix, all kept: 562 us in one order, 703 apart).
 static bool vsa_apart(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t kept, uint32_t splits,
                       uint32_t cus) {
   const uint32_t gen = 4 * cus;
