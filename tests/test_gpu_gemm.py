@@ -153,7 +153,7 @@ def check_against_exact_sums(dev, tokens, n, k):
     (1, 384, "few"), (32, 1152, "few"), (33, 384, "64x128"), (100, 8448, None),
     (200, 21504, "128x128 ring 2"), (520, 12288, "128x128 ring 2"), (1100, 21504, "128x128 ring 2"),
     (1500, 21504, "128x128 ring 2")])
-def test_every_tiling_of_a_short_k_is_bit_exact(dev, tokens, n, tiling, k):
+def test_every_tiling_is_bit_exact(dev, tokens, n, tiling, k):
     tiling = tiling or f"128x128 ring {4 if k >= 512 else 2}"
     assert gemm_tiling(tokens, n, k) == tiling
     check_against_exact_sums(dev, tokens, n, k)

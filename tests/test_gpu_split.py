@@ -17,13 +17,13 @@ pytestmark = pytest.mark.gpu
 
 
 # (tokens, token_count, query heads, key/value heads, pad) and the division, None for undivided or (blocks on
-# the undivided kernel, tiles per unit of the other full blocks, of the last, partial blocks): single calls
-# of one stage; two, three and seven stages (idle key groups); one key past eight stages; one to eight
-# live tiles in the last block; only whole blocks; a wave with no live row; units of two tiles; whole
-# rounds with the partial blocks, with a round of full blocks, and with both left over; head wrap and
-# padded output pitches
+# the undivided kernel, tiles per unit of the other full blocks, of the last, partial blocks): calls of one
+# stage, and of three whose units would be more than the chip holds; two, three and seven stages (idle key
+# groups); one key past eight stages; one to eight live tiles in the last block; only whole blocks; a wave
+# with no live row; units of two tiles; whole rounds with the partial blocks, with a round of full blocks, and
+# with both left over; head wrap and padded output pitches
 CASES = [
-    (1, 1, 2, 2, 0, None), (33, 33, 3, 3, 128, None),
+    (1, 1, 2, 2, 0, None), (33, 33, 3, 3, 128, None), (129, 129, 56, 56, 0, None),
     (65, 65, 2, 2, 0, (0, 1, 1)), (129, 129, 5, 5, 128, (0, 1, 1)), (257, 256, 8, 8, 0, (0, 1, 1)),
     (385, 385, 2, 2, 0, (0, 1, 1)), (447, 447, 3, 3, 0, (0, 1, 1)), (448, 448, 5, 5, 0, (0, 1, 1)),
     (449, 449, 3, 3, 0, (0, 1, 1)), (512, 449, 4, 2, 128, (0, 1, 1)), (513, 513, 4, 4, 0, (0, 1, 1)),
