@@ -35,18 +35,29 @@ CASES = [
     (34007, 34007, 2, 2, 0, (256, 1, 1))]
 
 
-def check_division(tokens, count, heads, plan):
-    got = split_plan(tokens, count, heads, H.capacity(tokens))
+def check_division(tokens, count, heads, plan, cap=None):
+    got = split_plan(tokens, count, heads, cap or H.capacity(tokens))
     assert got == plan, got
 
 
 @pytest.mark.parametrize("tokens,count,q_heads,kv_heads,pad,plan", CASES)
 def test_divided_calls_match_the_oracle_in_both_layouts(dev, tokens, count, q_heads, kv_heads, pad,
                                                         plan):
+    check_against_the_oracle(dev, tokens, count, q_heads, kv_heads, pad, plan, O.capacity(tokens))
+
+
+# capacities are multiples of 16, so V^T's rows begin at any 32 bytes of a 128-byte line: 96 (1,008 and 1,072),
+# 32 and, with no room for another token, 64
+@pytest.mark.parametrize("tokens,count,q_heads,kv_heads,cap", [
+    (1000, 1000, 7, 7, 1008), (1000, 999, 4, 2, 1040), (480, 480, 5, 5, 480), (1025, 1025, 3, 3, 1072)])
+def test_divided_calls_at_any_capacity(dev, tokens, count, q_heads, kv_heads, cap):
+    check_against_the_oracle(dev, tokens, count, q_heads, kv_heads, 0, (0, 1, 1), cap)
+
+
+def check_against_the_oracle(dev, tokens, count, q_heads, kv_heads, pad, plan, cap):
     import torch
 
-    check_division(tokens, count, q_heads, plan)
-    cap = O.capacity(tokens)
+    check_division(tokens, count, q_heads, plan, cap)
     rng = np.random.default_rng(tokens + 13 * q_heads)
     qc, qs, _, _, _ = head_major_operands(rng, q_heads, tokens, cap, late_match=False)
     _, _, kc, ks, vt = head_major_operands(rng, kv_heads, tokens, cap, late_match=False)
