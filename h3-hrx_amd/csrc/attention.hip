@@ -1160,11 +1160,11 @@ __device__ __forceinline__ void vsa_step(const char* kst, const char* vst, const
 
 __device__ __forceinline__ uint32_t rfl(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Query cubes that keep (nearly) every key cube: the prefix's. Their lists are several times a
+// Query cubes that keep (nearly) every key cube: the prefix's. Their lists can be several times a
 // video cube's (387 key cubes against 44 at 17,704 tokens behind a 154-token prefix, keep 10 %), and
 // a launch of one generation lasts as long as its longest list, so among the other cubes each of
-// them held up a whole generation (13 launches of 639 us there, 62 us without them). They go first,
-// in launches of their own, and where they are too few to fill the chip each is split: item
+// them held up a whole generation (13 launches of 639 us there, 62 us without them). Where it pays
+// (vsa_apart) they go first, in launches of their own, and where too few to fill the chip each is split: item
 // (cube, split) walks one range of the key cubes and writes its unnormalised O (f32 [64][128]) and
 // its rows' running max and sum, and k_vsa_combine weighs the ranges of a cube together.
 constexpr uint32_t kVsaPartO = 64 * 128;              // floats of an item's O
@@ -1739,7 +1739,7 @@ static uint32_t vsa_generation() { return std::max(1u, 4u * device_cus()); }
 // alone; apart, the prefix's ranges come first and every generation ends at `kept`. Of 560 runtime calls
 // timed both ways (13 to 923 key cubes, 1 to 40 heads, keep 2 to 99 %) 33 take the way that is slower by more
 // than 2 %, by 18 % at most (87 cubes of 16 heads, 21 of them prefix: 242 against 285 us); always apart 213 did,
-// by 48 % at most (112 cubes of 18 heads, 28 of them prefix, all kept: 562 us in one order, 703 apart).
+// by 48 % at most (67 cubes of 11 heads, 49 of them prefix: 223 us in one order, 330 apart).
 static bool vsa_apart(uint32_t heads, uint32_t cubes, uint32_t blocks, uint32_t kept, uint32_t splits,
                       uint32_t cus) {
   const uint32_t gen = 4 * cus;

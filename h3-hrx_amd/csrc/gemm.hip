@@ -24,7 +24,7 @@
 //
 // What bounds it: at full occupancy the matrix cores' power (54 % busy at an engine clock of 1.5 GHz,
 // 31,104 tokens: 1.95-2.05 POP/s against torch._int_mm's 2.10); with one tile per CU or fewer, what a
-// CU can load (about 21 bytes a clock) and the latency of a step.
+// CU can load (20 to 25 bytes a clock) and the latency of a step.
 #include <algorithm>
 #include <cmath>
 
